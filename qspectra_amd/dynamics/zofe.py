@@ -157,6 +157,8 @@ class ZOFEModel(DynamicalModel):
         Gamma = np.broadcast_to(Gamma, (P, S))
         w = np.broadcast_to(w, (P, S))
         flags = (1 if self.ham_hermit else 0) | (2 if self.rho_hermit else 0)
+        if not np.any(L * (1 - np.eye(N))):
+            flags |= 4                     # diagonal couplings (site occupations)
         eom = DeviceZOFE(H=_native.to_device(H, dev=dev), L=_native.to_device(L[None], dev=dev),
                          Gamma=_native.to_device(np.ascontiguousarray(Gamma)[None], dev=dev),
                          w=_native.to_device(np.ascontiguousarray(w)[None], dev=dev),
