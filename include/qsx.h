@@ -244,6 +244,36 @@ int32_t qsx_propagate_adjoint(const void* A, int64_t strideA, int32_t M, const v
                               int64_t workspace_bytes, void* gA, void* gy0, int32_t* status,
                               void* stream);
 
+/* The same propagation and its reverse mode for blocks of at most 16 elements,
+ * parallel in time: the N steps are cut into np = ceil(N / len) pieces of len
+ * steps (a power of two, 2..64), whose starts come from powers of P^len; the
+ * values equal the step-by-step recursion up to rounding.
+ *   A       [B|1][M][M] complex128 one-step propagators (strideA M^2 or 0)
+ *   y0      [B][R][M]
+ *   pos     int32 [nsave]: the step after which save s is taken, non-
+ *           decreasing, 0..N (0: y0 itself)
+ *   first   int32 [np + 1]: first[j] = number of saves with pos <= j len
+ *           (j < np), first[np] = nsave
+ *   v       [M] or null: with v (M <= 15) the saves are the signals v . y and
+ *           out and gout [B][R][nsave]; without, whole states [B][R][nsave][M]
+ *   Q, Y    [B|1][M][M] (P^len) and [B][R][np][M] (piece starts), written by
+ *           the forward call and read by the reverse one
+ *   gA [B][R][M][M], gy0 [B][R][M] (may be null): as qsx_propagate_adjoint
+ *   status  1: a non-finite state or gradient. */
+int32_t qsx_propagate_pieces(const void* A, int64_t strideA, int32_t M, const void* y0, int32_t R,
+                             int32_t B, const int32_t* pos, const int32_t* first, int32_t nsave,
+                             int64_t N, int32_t len, const void* v, void* Q, void* Y, void* out,
+                             int32_t* status, void* stream);
+int64_t qsx_propagate_pieces_adjoint_workspace_bytes(int32_t M, int32_t R, int32_t B, int64_t N,
+                                                     int32_t len);
+int32_t qsx_propagate_pieces_adjoint(const void* A, int64_t strideA, int32_t M, int32_t R,
+                                     int32_t B, const int32_t* pos, const int32_t* first,
+                                     int32_t nsave, int64_t N, int32_t len, const void* v,
+                                     const void* Q, const void* Y, const void* gout,
+                                     void* workspace, int64_t workspace_bytes, void* gA,
+                                     void* gy0, int32_t* status, void* stream);
+
+
 /* Linear-response signals of many problems of unequal size in one launch:
  * for problem b, y_{k+1} = P_b y_k from y0_b and s_k = v_b . y_k,
  * k = 0 .. nt-1, written to row r_b of out [B][nt] complex128 (FP64

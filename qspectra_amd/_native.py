@@ -39,6 +39,7 @@ c_i32, c_i64, c_dbl, c_vp, c_sz = (ctypes.c_int32, ctypes.c_int64, ctypes.c_doub
 
 # name -> argtypes (restype int32 unless listed in RESTYPES)
 RESTYPES = {'qsx_redfield_workspace_bytes': c_i64, 'qsx_heom_workspace_bytes': c_i64,
+            'qsx_propagate_pieces_adjoint_workspace_bytes': c_i64,
             'qsx_adjoint_workspace_bytes': c_i64, 'qsx_zofe_workspace_bytes': c_i64,
             'qsx_redfield_dense_workspace_bytes': c_i64, 'qsx_fourier_workspace_bytes': c_i64,
             'qsx_propagator_workspace_bytes': c_i64,
@@ -82,6 +83,12 @@ SIGNATURES = {
     'qsx_propagate_chunks': [c_i32, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i32, c_vp, c_i32,
                              c_i32, c_vp, c_vp, c_i32, c_vp, c_vp, c_vp],
     'qsx_adjoint_workspace_bytes': [c_i32, c_i32, c_i32, c_i64, c_i32],
+    'qsx_propagate_pieces': [c_vp, c_i64, c_i32, c_vp, c_i32, c_i32, c_vp, c_vp, c_i32, c_i64,
+                             c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp],
+    'qsx_propagate_pieces_adjoint_workspace_bytes': [c_i32, c_i32, c_i32, c_i64, c_i32],
+    'qsx_propagate_pieces_adjoint': [c_vp, c_i64, c_i32, c_i32, c_i32, c_vp, c_vp, c_i32, c_i64,
+                                     c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_vp,
+                                     c_vp, c_vp],
     'qsx_propagate_adjoint': [c_vp, c_i64, c_i32, c_vp, c_i32, c_i32, c_vp, c_i32, c_vp, c_i32,
                               c_vp, c_i64, c_vp, c_vp, c_vp, c_vp],
     'qsx_zgemm': [c_i32, c_i32, c_i32, c_i32, c_i32, c_dbl, c_dbl, c_vp, c_i64, c_i64, c_vp, c_i64,
@@ -642,6 +649,88 @@ def propagate_adjoint(A, y0, nsub, total_steps, gout, ckpt=64, stream=None):
                                        ptr(ws), ws.numel() * 16, ptr(gA), ptr(gy0), ptr(status),
                                        stream_ptr(stream))
     check(st, 'qsx_propagate_adjoint')
+    return gA, gy0, status
+
+
+MAX_PIECE_STATES = 16
+
+
+class PieceSchedule(object):
+    """Device tables of qsx_propagate_pieces for step counts nsub (host) of
+    the save intervals: the step after which each save is taken, cut into
+    pieces of ``len`` steps (the power of two next to sqrt(N), 8..64)."""
+
+    def __init__(self, nsub, dev):
+        pos = np.cumsum(np.maximum(np.asarray(nsub, dtype=np.int64).reshape(-1), 0))
+        self.N, self.nsave = int(pos[-1]), len(pos)
+        self.len = int(2 ** np.clip(np.ceil(np.log2(np.sqrt(max(self.N, 1)))), 3, 6))
+        self.np = -(-self.N // self.len)
+        first = np.searchsorted(pos, self.len * np.arange(self.np), side='right')
+        table = np.concatenate([pos, first, [self.nsave]]).astype(np.int32)
+        table = torch.as_tensor(table).to(dev)
+        self.pos, self.first = table[:self.nsave], table[self.nsave:]
+
+
+def _piece_operands(A, y0, sched, v):
+    B, R, M = y0.shape
+    if A.dtype != torch.complex128 or y0.dtype != torch.complex128:
+        raise TypeError('propagate_pieces needs complex128 operands')
+    if A.shape[-2:] != (M, M) or A.shape[0] not in (1, B):
+        raise ValueError('operator shape %s does not match states %s' % (tuple(A.shape),
+                                                                          tuple(y0.shape)))
+    if M > MAX_PIECE_STATES - (v is not None) or sched.N < 1:
+        raise ValueError('propagate_pieces: %d states, %d steps' % (M, sched.N))
+    if v is not None and (v.dtype != torch.complex128 or tuple(v.shape) != (M,)):
+        raise ValueError('propagate_pieces: signal vector of shape %s' % (tuple(v.shape),))
+    return A.contiguous(), y0.contiguous(), None if v is None else v.contiguous()
+
+
+def propagate_pieces(A, y0, sched, v=None, stream=None):
+    """qsx_propagate_pieces: (out, Q, Y, status) for y <- A y from y0
+    [B, R, M] over a PieceSchedule: states out [B, R, nsave, M], or the
+    signals v . y [B, R, nsave]; Q and Y are what the reverse call needs."""
+    lib = require_native()
+    A, y0, v = _piece_operands(A, y0, sched, v)
+    B, R, M = y0.shape
+    kw = dict(dtype=torch.complex128, device=y0.device)
+    out = torch.empty((B, R, sched.nsave) + (() if v is not None else (M,)), **kw)
+    Q = torch.empty((A.shape[0], M, M), **kw)
+    Y = torch.empty((B, R, sched.np, M), **kw)
+    status = torch.zeros(1, dtype=torch.int32, device=y0.device)
+    with timing.launch('pieces M=%d R=%d B=%d steps=%d len=%d' % (M, R, B, sched.N, sched.len),
+                       stream):
+        st = lib.qsx_propagate_pieces(ptr(A), 0 if A.shape[0] == 1 else M * M, M, ptr(y0), R, B,
+                                      ptr(sched.pos), ptr(sched.first), sched.nsave, sched.N,
+                                      sched.len, ptr(v), ptr(Q), ptr(Y), ptr(out), ptr(status),
+                                      stream_ptr(stream))
+    check(st, 'qsx_propagate_pieces')
+    return out, Q, Y, status
+
+
+def propagate_pieces_adjoint(A, y0, sched, Q, Y, gout, v=None, stream=None):
+    """qsx_propagate_pieces_adjoint: (gA [B, R, M, M], gy0 [B, R, M], status)
+    from the cotangents gout of propagate_pieces' out."""
+    lib = require_native()
+    A, y0, v = _piece_operands(A, y0, sched, v)
+    B, R, M = y0.shape
+    if tuple(gout.shape) != (B, R, sched.nsave) + (() if v is not None else (M,)):
+        raise ValueError('cotangents of shape %s' % (tuple(gout.shape),))
+    gout = gout.contiguous()
+    nbytes = lib.qsx_propagate_pieces_adjoint_workspace_bytes(M, R, B, sched.N, sched.len)
+    if nbytes < 0:
+        raise NativeError('invalid adjoint workspace request')
+    kw = dict(dtype=torch.complex128, device=y0.device)
+    ws = torch.empty((nbytes + 15) // 16, **kw)
+    gA = torch.empty((B, R, M, M), **kw)
+    gy0 = torch.empty((B, R, M), **kw)
+    status = torch.zeros(1, dtype=torch.int32, device=y0.device)
+    with timing.launch('pieces adjoint M=%d R=%d B=%d steps=%d len=%d'
+                       % (M, R, B, sched.N, sched.len), stream):
+        st = lib.qsx_propagate_pieces_adjoint(
+            ptr(A), 0 if A.shape[0] == 1 else M * M, M, R, B, ptr(sched.pos), ptr(sched.first),
+            sched.nsave, sched.N, sched.len, ptr(v), ptr(Q), ptr(Y), ptr(gout), ptr(ws),
+            ws.numel() * 16, ptr(gA), ptr(gy0), ptr(status), stream_ptr(stream))
+    check(st, 'qsx_propagate_pieces_adjoint')
     return gA, gy0, status
 
 

@@ -134,6 +134,13 @@ __device__ inline float dpp_move(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
+// Lane I of each 16-lane row of v, broadcast to the row (DPP row_newbcast,
+// one move of 64 bits; the row's lanes must all be active).
+template <int I>
+__device__ __forceinline__ double row_lane(double v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + I, 0xF, 0xF, true);
+}
+
 // Sum over aligned segments of S lanes (S = 1, 2, 4, 8 or 16); every lane of
 // a segment receives the same total.  Butterfly over quad permutations
 // [1,0,3,2] and [2,3,0,1], then the half-row and row mirrors (lane i with

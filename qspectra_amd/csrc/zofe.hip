@@ -415,12 +415,6 @@ inline size_t zofe_column_lds_bytes(int N, int S, int P) {
          (size_t)N * (S + 1) * sizeof(int);
 }
 
-// Lane I of each 16-lane row, broadcast to the row (every lane active).
-template <int I>
-__device__ __forceinline__ double row_lane(double v) {
-  return __builtin_amdgcn_update_dpp(v, v, 0x150 + I, 0xF, 0xF, true);
-}
-
 // d[c][i] += be[i][k] x[c] for i = I .. N - 1, be[i][k] held by lane i
 template <int I, int N, int C>
 struct ColumnFma {

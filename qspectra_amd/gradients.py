@@ -70,6 +70,33 @@ class _Propagate(torch.autograd.Function):
         return gA, gy0, None, None
 
 
+class _PropagatePieces(torch.autograd.Function):
+    """The map of _Propagate for blocks of at most 16 states, parallel in
+    time (qsx_propagate_pieces and its reverse mode): states
+    [B, R, nsave, M], or with a constant vector v the signals v . y
+    [B, R, nsave]."""
+
+    @staticmethod
+    def forward(ctx, A, y0, sched, v):
+        out, Q, Y, status = _native.propagate_pieces(A, y0, sched, v)
+        ctx.save_for_backward(A, y0, Q, Y, v)
+        ctx.sched = sched
+        ctx.mark_non_differentiable(status)
+        return out, status
+
+    @staticmethod
+    def backward(ctx, gout, _gstatus):
+        A, y0, Q, Y, v = ctx.saved_tensors
+        gA, gy0, status = _native.propagate_pieces_adjoint(A, y0, ctx.sched, Q, Y, gout, v)
+        if int(status.item()) != 0:
+            raise FloatingPointError('adjoint propagation failed (status %d)'
+                                     % int(status.item()))
+        gA = gA.sum(dim=1)
+        if A.shape[0] == 1 and gA.shape[0] > 1:
+            gA = gA.sum(dim=0, keepdim=True)
+        return gA, gy0, None, None
+
+
 class _RK4Propagator(torch.autograd.Function):
     """P = P4(h L) = I + hL + (hL)^2/2 + (hL)^3/6 + (hL)^4/24 for L [B, M, M].
 
@@ -109,12 +136,36 @@ def rk4_propagator(L, h):
     return _RK4Propagator.apply(L, h)
 
 
+# steps from which the recursion is cut into pieces: below, a chain of N steps
+# is no longer than the pieces' extra launches
+PIECE_STEPS = 64
+# memory of the reverse pass's partial gradients (one M x M block per piece):
+# beyond it, right-hand sides alone fill the chip
+PIECE_BYTES = 1 << 29
+
+
+def _pieces(M, rhs, nsub, dev, signal=False):
+    """The PieceSchedule serving rhs right-hand sides of M states over the
+    save intervals nsub, or None where the step-by-step recursion does."""
+    if M > _native.MAX_PIECE_STATES - bool(signal):
+        return None
+    if not PIECE_STEPS <= int(np.sum(np.maximum(nsub, 0))) < 1 << 24:
+        return None
+    sched = _native.PieceSchedule(nsub, dev)
+    return sched if 16 * rhs * sched.np * M * (M + 2) <= PIECE_BYTES else None
+
+
 def propagate(A, y0, nsub, ckpt=64):
     """Differentiable propagation with the one-step propagator A [B|1, M, M]:
     states [B, R, len(nsub), M] (nsub: host step counts per save interval).
     The reverse pass recomputes the forward states from checkpoints every
-    ckpt steps (blocks up to M = 160)."""
-    states, status = _Propagate.apply(A, y0, nsub, int(ckpt))
+    ckpt steps (blocks up to M = 160; at most 16 states: from the starts of
+    the pieces the steps are cut into, see _native.PieceSchedule)."""
+    sched = _pieces(y0.shape[-1], y0.shape[0] * y0.shape[1], nsub, y0.device)
+    if sched is not None:
+        states, status = _PropagatePieces.apply(A, y0, sched, None)
+    else:
+        states, status = _Propagate.apply(A, y0, nsub, int(ckpt))
     if int(status.item()) != 0:
         raise FloatingPointError('propagation produced a non-finite state')
     return states
@@ -225,6 +276,8 @@ class RedfieldAbsorption(object):
             self.size, 1, -1).contiguous()
         self.nsub = np.ones(len(self.t), dtype=np.int64)
         self.nsub[0] = 0
+        # signals straight from the propagation, in pieces of the time grid
+        self._pieces = _pieces(self.N, self.size, self.nsub, dev, signal=True)
 
     def hamiltonians(self, E, J):
         H = site_hamiltonian(E, J)
@@ -245,6 +298,11 @@ class RedfieldAbsorption(object):
         H1 = self.hamiltonians(E, J)
         L = self.liouvillian(H1, lam)
         P = rk4_propagator(L, self.dt)
+        if self._pieces is not None:
+            x, status = _PropagatePieces.apply(P, self.y0, self._pieces, self.v)
+            if int(status.item()) != 0:
+                raise FloatingPointError('propagation produced a non-finite state')
+            return x[:, 0].mean(dim=0)
         states = propagate(P, self.y0, self.nsub, self.ckpt)       # [B, 1, nt, M]
         x = torch.einsum('bkm,m->bk', states[:, 0], self.v)
         return x.mean(dim=0)
