@@ -420,12 +420,11 @@ def _reference_default_err():
 # HEOM bytes per state element and RK4 step.  Algorithmic: four stages each
 # reading and writing the stage operand (16 B FP64, 8 B MIXED) plus one read
 # and one write of the FP64 state: 160 / 96 B.  The stage kernel as written
-# moves more (no accumulator buffer): FP64 reads y in stages 2..4 and the
-# stage vectors z2, z3 again in stage 4 (48 + 48 + 48 + 64 = 208 B); MIXED
-# writes the stage derivatives k1..k3 in complex64 and reads them, the FP64
-# state and the complex64 copy of y back (24 + 32 + 32 + 72 = 160 B).
+# moves more: it writes the terms v1..v3 of the step's polynomial and reads v1,
+# v2 and y again in stage 4 (FP64 32 + 32 + 32 + 80 = 176 B; MIXED, terms in
+# complex64 and y in FP64, 24 + 16 + 16 + 56 = 112 B).
 HEOM_ALGORITHMIC_BYTES = {'fp64': 160, 'mixed': 96}
-HEOM_BYTES_PER_ELEMENT_STEP = {'fp64': 208, 'mixed': 160}
+HEOM_BYTES_PER_ELEMENT_STEP = {'fp64': 176, 'mixed': 112}
 
 # HBM bytes per launch (read + written) measured with rocprofv3 --pmc
 # FETCH_SIZE and WRITE_SIZE over the `bench.py --counters` sequence, FETCH
@@ -436,9 +435,10 @@ HEOM_BYTES_PER_ELEMENT_STEP = {'fp64': 208, 'mixed': 160}
 # launch of several kernels counts all of them.
 PMC_TRAFFIC = {
     # one RK4 stage over 256 members, summed over its sample passes (10 of 24
-    # members and one of 16; FP64 70.8 B per element-stage, MIXED 50.4 B)
-    'heom stage fp64': 2.718e9,
-    'heom stage mixed': 1.936e9,
+    # members and one of 16 in FP64, 6 of 40 and one of 16 in MIXED; FP64 58.6 B
+    # per element-stage, MIXED 37.0 B)
+    'heom stage fp64': 2.251e9,
+    'heom stage mixed': 1.421e9,
     # the headline plan's t2 operator program (one work-group, M = 49)
     'propagate powers M=49 B=1 R=7 e=0,100,200,500': 8.64e4,
     'chunks prop mixed M=147 nc=8 B=1 steps=15 nsave=16': 4.30e6,

@@ -25,15 +25,19 @@
 // -i unit (H_X rho - rho H_Y) with the Hilbert blocks H_X (nX x nX) and H_Y
 // (nY x nY): nX + nY instead of M products per element.
 //
-// One RK4 stage is one launch over (sample, ADO tile).  Classical RK4 is
-// stored without an update accumulator: with z1 = y, z2 = y + h/2 k1,
-// z3 = y + h/2 k2, z4 = y + h k3, the step is
-//   y' = y + ((z2 - y) + 2 (z3 - y) + (z4 - y)) / 3 + h/6 k4,
-// so FP64 keeps y and the stage vectors z2, z3, z4 (208 bytes per element
-// and step instead of 288 with a separate accumulator).  MIXED keeps the
-// stage vectors and the stage derivatives k1..k3 in complex64 (a complex64
-// copy z1 of the state serves the neighbour gathers of stage 1) and forms
-// y' = y + h/6 (k1 + 2 k2 + 2 k3 + k4) in FP64 (160 bytes instead of 224).
+// One RK4 stage is one launch over (sample, ADO tile).  Without fields the
+// generator A does not depend on time, and a classical RK4 step is exactly
+//   y' = y + v1 + v2 + v3 + v4,   v1 = h A y,  v_{k+1} = h/(k+1) A v_k,
+// so a stage reads its input and writes the next term, and only the last one
+// reads y, v1 and v2 again: 176 bytes per element and step in FP64 (208 with
+// stage vectors y + c h k), 112 in MIXED (160), which holds y in FP64 (the
+// first stage gathers it so) and the terms in complex64.  With fields
+// the stages see different generators: z1 = y, z2 = y + h/2 k1, z3 = y + h/2
+// k2, z4 = y + h k3, and
+//   y' = y + ((z2 - y) + 2 (z3 - y) + (z4 - y)) / 3 + h/6 k4
+// from the stage vectors in FP64; MIXED keeps the stage vectors and the stage
+// derivatives k1..k3 in complex64 and forms y' = y + h/6 (k1 + 2 k2 + 2 k3 +
+// k4) in FP64.
 // Work-groups are mapped so that every tile of one sample lands on the same
 // XCD (work-groups are dispatched round-robin over the 8 XCDs): a sample's
 // hierarchy and its neighbour re-reads stay in one L2.
@@ -77,6 +81,12 @@ struct HeomArgs {
   const int* rsite;        // [M][nrel] sites occupied in the row or column state (-1 pad)
   const double* rocc;      // [M][nrel][2] their occupations (row, column)
 };
+
+// acc += i b z
+__device__ inline void imag_fma(double2& acc, double b, double2 z) {
+  acc.x = fma(-b, z.y, acc.x);
+  acc.y = fma(b, z.x, acc.y);
+}
 
 template <typename T>
 __device__ inline double2 ld(const cplx_t<T>* p) { return to_d2(*p); }
@@ -146,10 +156,12 @@ __device__ inline double2 neighbour_sum(const HeomArgs& a, const int* ts, const 
 }
 
 // Buffers of the RK4 stages (see the file comment): y the FP64 state, z[1..3]
-// the stage vectors z2..z4, z[0] the complex64 copy of y (MIXED only), k the
-// complex64 stage derivatives k1..k3 (MIXED only).
+// the terms v1..v3 (series) or the stage vectors z2..z4; with stage vectors in
+// MIXED z[0] the complex64 copy of y and k the complex64 stage derivatives
+// k1..k3.
 template <typename T>
 struct HeomStageBufs {
+  bool series;
   double2* y;
   cplx_t<T>* z[4];
   cplx_t<T>* k[3];
@@ -157,13 +169,25 @@ struct HeomStageBufs {
 
 // The stage's output for element gi given its derivative k = F(zin)[gi] and
 // zp = zin[gi] (see the file comment for the buffers): st = 4 writes
-// zout = k; otherwise the RK4 stage st.
+// zout = k; otherwise the RK4 stage st (h: the step, or in the series the
+// step over st + 1).
 template <typename T>
 __device__ __forceinline__ void stage_epilogue(double2 k, double2 zp, int64_t gi, int st, double h,
                                                const HeomStageBufs<T>& bf,
                                                cplx_t<T>* __restrict__ zout) {
   if (st == 4) {                           // plain application: zout = F(zin)
     zout[gi] = from_d2<T>(k);
+    return;
+  }
+  if (bf.series) {
+    const double2 v = make_double2(h * k.x, h * k.y);
+    if (st < 3) {                          // the next term
+      bf.z[st + 1][gi] = from_d2<T>(v);
+      return;
+    }
+    const double2 yv = bf.y[gi], v1 = ld<T>(bf.z[1] + gi), v2 = ld<T>(bf.z[2] + gi);
+    const double2 yn = cadd(yv, cadd(v1, cadd(v2, cadd(zp, v))));
+    bf.y[gi] = yn;
     return;
   }
   if constexpr (std::is_same<T, double>::value) {
@@ -201,9 +225,10 @@ __device__ __forceinline__ void stage_epilogue(double2 k, double2 zp, int64_t gi
 // shape, edge by edge.
 template <typename T, int NR, int KB>
 __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
-    HeomArgs a, const cplx_t<T>* __restrict__ zin, cplx_t<T>* __restrict__ zout,
+    HeomArgs a, const void* __restrict__ zin_, cplx_t<T>* __restrict__ zout,
     HeomStageBufs<T> bf, double h, int st) {
   using T2 = cplx_t<T>;
+  const T2* __restrict__ zin = static_cast<const T2*>(zin_);
   extern __shared__ __align__(16) unsigned char smem[];
   const int opsz = heom_opsz(a);
   const int nb2 = 2 * a.nbins;
@@ -310,19 +335,29 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // stage as heom_stage_kernel with every index division by a constant, the
 // 2 (NX + NY) commutator terms unrolled with LDS offsets fixed at compile
 // time, and the per-element neighbour weights (site bin, n_j(r) - n_j(c),
-// c_k n_j(r) - conj(c_k) n_j(c)) tabulated once per work-group.  Absent
-// edges point at the element's own ADO with a zero coefficient, so the
-// gathers need no tests.  Counters on the 7-site, 3060-ADO hierarchy showed
-// the generic kernel issuing ~490 vector instructions per element (the
-// vector units busy 60% of the launch); this one issues about half as many,
-// which made the MIXED stage 13% faster and the FP64 stage 2-5%: what is
-// left is the latency of the neighbour gathers at four waves per SIMD (the
-// 120 registers; forcing six or eight waves spills).
-template <typename T, int NX, int NY, int NR, int KB>
-__global__ __launch_bounds__(kThreads) void heom_comm_kernel(
-    HeomArgs a, const cplx_t<T>* __restrict__ zin, cplx_t<T>* __restrict__ zout,
+// c_k n_j(r) - conj(c_k) n_j(c)) tabulated once per work-group.
+// Three quarters of the (ADO, bin, kind) edges of a truncated hierarchy do not
+// exist (no upward ones at the last level, downward ones only from occupied
+// bins): their gathers, coefficients and products are skipped lane by lane.
+// Purely imaginary operators (-i unit H of a real H, -i unit times a real
+// edge coefficient) take half the multiply-adds; the form is decided per
+// work-group from the entries it has loaded.
+// Measured (7 sites, 3060 ADOs, per stage of 24 samples): 49 us FP64, 47 us
+// MIXED; 74 and 66 us when every edge was gathered, all products were complex
+// and stages wrote separate stage vectors (55 and 62 us with the existing
+// edges alone).  In FP64 a stage now moves 210 MB (FETCH_SIZE, WRITE_SIZE) at
+// 4.3 TB/s, where a device copy reaches 5.1.  Six wavefronts per SIMD (a few
+// spilled registers) beat five by 3% and 8%; holding an element's operator
+// entries in registers, nested brackets y + h/m A (..) in place of the series
+// terms, and non-temporal loads and stores were slower.
+// TIN: the type of the stage's input (MIXED: double for the series' first
+// stage, whose input is y).
+template <typename T, typename TIN, int NX, int NY, int NR, int KB>
+__global__ __launch_bounds__(kThreads, KB == 2 ? 6 : 4) void heom_comm_kernel(
+    HeomArgs a, const void* __restrict__ zin_, cplx_t<T>* __restrict__ zout,
     HeomStageBufs<T> bf, double h, int st) {
-  using T2 = cplx_t<T>;
+  using T2 = cplx_t<TIN>;
+  const T2* __restrict__ zin = static_cast<const T2*>(zin_);
   constexpr int M = NX * NY;
   constexpr int OPSZ = NX == NY ? NX * NX : NX * NX + NY * NY;
   __shared__ int pbin[M][NR];           // 2 * (first bin of the slot's site)
@@ -331,8 +366,8 @@ __global__ __launch_bounds__(kThreads) void heom_comm_kernel(
   extern __shared__ __align__(16) unsigned char smem[];
   const int nb2 = 2 * a.nbins;
   double2* Hs = reinterpret_cast<double2*>(smem);
-  T2* zt = reinterpret_cast<T2*>(Hs + OPSZ);
-  size_t off = (size_t)OPSZ * sizeof(double2) + (size_t)a.ado_per_tile * M * sizeof(T2);
+  double2* zt = Hs + OPSZ;
+  size_t off = ((size_t)OPSZ + (size_t)a.ado_per_tile * M) * sizeof(double2);
   off = (off + 15) & ~(size_t)15;
   double2* tcf = reinterpret_cast<double2*>(smem + off);
   int* tsrc = reinterpret_cast<int*>(tcf + a.ado_per_tile * nb2);
@@ -352,14 +387,19 @@ __global__ __launch_bounds__(kThreads) void heom_comm_kernel(
   const int nloc = min(a.ado_per_tile, a.n_ado - ado0);
   const int64_t base = ((int64_t)b * a.n_ado + ado0) * M;
   const double2* Hb = a.Hop + (int64_t)b * OPSZ;
-  for (int e = tid; e < OPSZ; e += kThreads) Hs[e] = Hb[e];
-  for (int e = tid; e < nloc * M; e += kThreads) zt[e] = zin[base + e];
+  bool general = false;                      // operators not purely imaginary
+  for (int e = tid; e < OPSZ; e += kThreads) {
+    Hs[e] = Hb[e];
+    general |= Hs[e].x != 0.0;
+  }
+  for (int e = tid; e < nloc * M; e += kThreads) zt[e] = ld<TIN>(zin + base + e);
   for (int e = tid; e < nloc * nb2; e += kThreads) {
     const int64_t g = (int64_t)ado0 * nb2 + e;
     const int src = a.bsrc[g];
     const bool ok = src >= 0 && src < a.n_ado;
-    tsrc[e] = ok ? src : ado0 + e / nb2;
+    tsrc[e] = ok ? src : -1;
     tcf[e] = ok ? a.bcoef[g] : make_double2(0.0, 0.0);
+    general |= tcf[e].x != 0.0;
   }
   for (int e = tid; e < M * NR; e += kThreads) {
     const int p = e / NR, t = e % NR;
@@ -375,68 +415,95 @@ __global__ __launch_bounds__(kThreads) void heom_comm_kernel(
       pwm[p][t][kk] = make_double2(c.x * orow - c.x * ocol, c.y * orow + c.y * ocol);
     }
   }
-  __syncthreads();
+  general = __syncthreads_or(general);
 
   const double2* HY = NX == NY ? Hs : Hs + NX * NX;   // square blocks: H_Y = H_X
   const T2* zb = zin + (int64_t)b * a.n_ado * M;
-  for (int e = tid; e < nloc * M; e += kThreads) {
-    const int la = e / M, p = e - la * M, ado = ado0 + la;
-    const int r = p % NX, c = p / NX;
-    const T2* z = zt + la * M;
-    // (H_X rho - rho H_Y)_{rc}, p = r + NX c, column-major rho
-    double2 k = make_double2(0.0, 0.0);
+  auto elements = [&](auto form) {
+    constexpr bool GENERAL = decltype(form)::value;
+    for (int e = tid; e < nloc * M; e += kThreads) {
+      const int la = e / M, p = e - la * M, ado = ado0 + la;
+      const int r = p % NX, c = p / NX;
+      const double2* z = zt + la * M;
+      // per occupied-site slot: the neighbour gathers of the edges that exist,
+      // in flight during a half of the commutator
+      const double2* tc = tcf + la * nb2;
+      const double2 zp = z[p];
+      double2 k = cmul(make_double2(a.shift[ado] + a.dvec[p].x, a.dvec[p].y), zp);
 #pragma unroll
-    for (int q = 0; q < NX; ++q) k = cadd(k, cmul(Hs[r * NX + q], ld<T>(z + q + NX * c)));
+      for (int t = 0; t < NR; ++t) {
+        const int2* ts = reinterpret_cast<const int2*>(tsrc + la * nb2 + pbin[p][t]);
+        int src[2 * KB];
+        T2 v[2 * KB];
 #pragma unroll
-    for (int q = 0; q < NY; ++q) {
-      const double2 t = cmul(ld<T>(z + r + NX * q), HY[q * NY + c]);
-      k.x -= t.x;
-      k.y -= t.y;
-    }
-    const double2 zp = ld<T>(z + p);
-    const double2 dg = make_double2(a.shift[ado] + a.dvec[p].x, a.dvec[p].y);
-    k = cadd(k, cmul(dg, zp));
-    // neighbour terms: all offsets and weights, then all gathers, then the sum
-    const int* ts = tsrc + la * nb2;
-    const double2* tc = tcf + la * nb2;
-    constexpr int NE = 2 * NR * KB;
-    int src[NE];
-    double2 w[NE];
+        for (int kk = 0; kk < KB; ++kk) {
+          const int2 sk = ts[kk];
+          src[2 * kk] = sk.x;
+          src[2 * kk + 1] = sk.y;
+        }
 #pragma unroll
-    for (int t = 0; t < NR; ++t) {
-      const int b0 = pbin[p][t];
-      const double wp = pwp[p][t];
+        for (int o = 0; o < 2 * KB; ++o) {
+          v[o] = T2{0, 0};
+          if (src[o] >= 0) v[o] = zb[src[o] * M + p];
+        }
+        // (H_X rho - rho H_Y)_{rc}, p = r + NX c, column-major rho
+        if (t == 0) {
 #pragma unroll
-      for (int kk = 0; kk < KB; ++kk) {
-        const int bi = b0 + 2 * kk, e0 = 2 * (t * KB + kk);
-        src[e0] = ts[bi];
-        src[e0 + 1] = ts[bi + 1];
-        const double2 c0 = tc[bi];
-        w[e0] = make_double2(c0.x * wp, c0.y * wp);
-        w[e0 + 1] = cmul(tc[bi + 1], pwm[p][t][kk]);
+          for (int q = 0; q < NX; ++q) {
+            const double2 x = z[q + NX * c];
+            if (GENERAL) cfma<double>(k, Hs[r * NX + q], x);
+            else imag_fma(k, Hs[r * NX + q].y, x);
+          }
+        }
+        if (t == NR - 1) {
+#pragma unroll
+          for (int q = 0; q < NY; ++q) {
+            const double2 x = z[r + NX * q];
+            if (GENERAL) cfma<double>(k, make_double2(-x.x, -x.y), HY[q * NY + c]);
+            else imag_fma(k, -HY[q * NY + c].y, x);
+          }
+        }
+#pragma unroll
+        for (int o = 0; o < 2 * KB; ++o) {
+          if (src[o] >= 0) {
+            const double2 cf = tc[pbin[p][t] + o], x = to_d2(v[o]);
+            if (o % 2 == 0) {
+              const double w = pwp[p][t];
+              if (GENERAL) cfma<double>(k, make_double2(cf.x * w, cf.y * w), x);
+              else imag_fma(k, cf.y * w, x);
+            } else {
+              const double2 wm = pwm[p][t][o / 2];
+              cfma<double>(k, GENERAL ? cmul(cf, wm) : make_double2(-cf.y * wm.y, cf.y * wm.x),
+                           x);
+            }
+          }
+        }
       }
+      stage_epilogue<T>(k, zp, base + e, st, h, bf, zout);
     }
-    T2 v[NE];
-#pragma unroll
-    for (int q = 0; q < NE; ++q) v[q] = zb[src[q] * M + p];
-#pragma unroll
-    for (int q = 0; q < NE; ++q) k = cadd(k, cmul(w[q], to_d2(v[q])));
-    stage_epilogue<T>(k, zp, base + e, st, h, bf, zout);
-  }
+  };
+  if (general) elements(std::true_type());
+  else elements(std::false_type());
 }
 
 template <typename T>
-using StageKernel = void (*)(HeomArgs, const cplx_t<T>*, cplx_t<T>*, HeomStageBufs<T>, double,
+using StageKernel = void (*)(HeomArgs, const void*, cplx_t<T>*, HeomStageBufs<T>, double,
                              int);
+
+// whether heom_comm_kernel serves the hierarchy
+inline bool is_comm_shape(const HeomArgs& a) {
+  return !a.dense && a.N == 0 && a.nX == a.nY && a.nX >= 2 && a.nX <= 8 && a.nrel == 2 &&
+         (a.K1 == 2 || a.K1 == 3);
+}
 
 // the stage kernel for the hierarchy's neighbour shape (occupied-site slots
 // per element, bins per site)
-template <typename T>
+template <typename T, typename TIN = T>
 StageKernel<T> pick_stage_kernel(const HeomArgs& a) {
-  if (!a.dense && a.N == 0 && a.nX == a.nY && a.nrel == 2 && (a.K1 == 2 || a.K1 == 3)) {
+  if (is_comm_shape(a)) {
 #define QSX_COMM(n_)                                                               \
-    if (a.nX == n_) return a.K1 == 2 ? heom_comm_kernel<T, n_, n_, 2, 2>           \
-                                     : heom_comm_kernel<T, n_, n_, 2, 3>;
+    if (a.nX == n_) return a.K1 == 2 ? heom_comm_kernel<T, TIN, n_, n_, 2, 2>      \
+                                     : heom_comm_kernel<T, TIN, n_, n_, 2, 3>;
     QSX_COMM(2) QSX_COMM(3) QSX_COMM(4) QSX_COMM(5) QSX_COMM(6) QSX_COMM(7) QSX_COMM(8)
 #undef QSX_COMM
   }
@@ -519,9 +586,12 @@ inline int heom_samples_per_pass(int B, int64_t bytes_per_sample) {
   return std::min(B, c);
 }
 
-// workspace bytes per hierarchy element: FP64 y, z2, z3, z4; MIXED y and the
-// complex64 z1..z4, k1..k3
-inline int64_t heom_bytes_per_element(bool fp64) { return fp64 ? 4 * 16 : 16 + 7 * 8; }
+// workspace bytes per hierarchy element: FP64 y and three terms or stage
+// vectors; MIXED y and in complex64 three terms, or with stage vectors its
+// copy, z2..z4 and k1..k3
+inline int64_t heom_bytes_per_element(bool fp64, bool series) {
+  return fp64 ? 4 * 16 : 16 + (series ? 3 : 7) * 8;
+}
 
 template <typename T>
 int run_heom(const HeomArgs& a0, const double2* y0, const int32_t* nsub, const double* h,
@@ -530,25 +600,32 @@ int run_heom(const HeomArgs& a0, const double2* y0, const int32_t* nsub, const d
   using T2 = cplx_t<T>;
   constexpr bool kFp64 = std::is_same<T, double>::value;
   const int64_t per = (int64_t)a0.n_ado * a0.M;               // elements per sample
-  const int Bc = heom_samples_per_pass(a0.B, per * heom_bytes_per_element(kFp64));
+  // MIXED outside the commutator kernel keeps the stage vectors (the other
+  // kernels read their input in complex64)
+  const bool series = fl.P == 0 && (kFp64 || is_comm_shape(a0));
+  const int Bc = heom_samples_per_pass(a0.B, per * heom_bytes_per_element(kFp64, series));
   const int64_t ctotal = (int64_t)Bc * per;
   HeomStageBufs<T> bf;
+  bf.series = series;
   bf.y = static_cast<double2*>(workspace);
   T2* zbase = reinterpret_cast<T2*>(bf.y + ctotal);
-  bf.z[0] = kFp64 ? nullptr : zbase;
-  T2* zn = kFp64 ? zbase : zbase + ctotal;
+  bf.z[0] = kFp64 || series ? nullptr : zbase;
+  T2* zn = kFp64 || series ? zbase : zbase + ctotal;
   for (int i = 1; i < 4; ++i) bf.z[i] = zn + (i - 1) * ctotal;
-  for (int i = 0; i < 3; ++i) bf.k[i] = kFp64 ? nullptr : zn + (3 + i) * ctotal;
-  // the stage inputs: y itself (FP64) or its complex64 copy, then z2..z4
-  const T2* zins[4] = {kFp64 ? reinterpret_cast<const T2*>(bf.y) : bf.z[0], bf.z[1], bf.z[2],
-                       bf.z[3]};
+  for (int i = 0; i < 3; ++i) bf.k[i] = kFp64 || series ? nullptr : zn + (3 + i) * ctotal;
+  // the stage inputs: y itself or (stage vectors in MIXED) its complex64 copy,
+  // then z[1..3]
+  const void* zins[4] = {kFp64 || series ? (const void*)bf.y : bf.z[0], bf.z[1], bf.z[2], bf.z[3]};
   const int opsz = heom_opsz(a0);
-  const size_t shmem = heom_lds_bytes(opsz, a0.ado_per_tile, a0.M, a0.nbins, sizeof(T2), a0.N);
+  const size_t shmem = heom_lds_bytes(opsz, a0.ado_per_tile, a0.M, a0.nbins,
+                                       is_comm_shape(a0) ? sizeof(double2) : sizeof(T2), a0.N);
   QSX_CHECK_ARG(shmem <= 160 * 1024, "qsx_heom_propagate: %zu bytes of LDS", shmem);
   const StageKernel<T> kern = pick_stage_kernel<T>(a0);
+  const StageKernel<T> first = series ? pick_stage_kernel<T, double>(a0) : kern;
   if (shmem > 64 * 1024)
-    QSX_CHECK_HIP(hipFuncSetAttribute((const void*)kern,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
+    for (const StageKernel<T> k : {kern, first})
+      QSX_CHECK_HIP(hipFuncSetAttribute((const void*)k,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
   static const int kStageSample[4] = {0, 1, 1, 2};   // t, t + h/2, t + h/2, t + h
   for (int b0 = 0; b0 < a0.B; b0 += Bc) {
     HeomArgs a = a0;
@@ -574,8 +651,9 @@ int run_heom(const HeomArgs& a0, const double2* y0, const int32_t* nsub, const d
                                fl.C + (int64_t)b0 * fl.strideC, fl.strideC,
                                fl.F + (int64_t)b0 * fl.strideF, fl.strideF, g,
                                kStageSample[st], fl.P, a.B, opsz, fl.Hwork);
-          hipLaunchKernelGGL(kern, dim3(ngroups), dim3(kThreads), shmem, stream, a, zins[st],
-                             (T2*)nullptr, bf, h[s], st);
+          hipLaunchKernelGGL(st == 0 ? first : kern, dim3(ngroups), dim3(kThreads), shmem, stream,
+                             a, zins[st],
+                             (T2*)nullptr, bf, bf.series ? h[s] / (st + 1) : h[s], st);
         }
         ++g;
       }
@@ -627,8 +705,13 @@ static int fill_args(qsx::HeomArgs& a, int B, int n_ado, int M, int n, const voi
   a.nbins = nbins;
   a.K1 = K1;
   a.nrel = nrel;
-  a.ado_per_tile = std::max(1, kElemsPerThread * kThreads / M);
-  a.tiles = (n_ado + a.ado_per_tile - 1) / a.ado_per_tile;
+  // fewer elements per thread while the launch would not give every CU two
+  // work-groups (one 3060-ADO hierarchy: 204 work-groups at 3, 612 at 1)
+  for (int elems = kElemsPerThread; elems >= 1; --elems) {
+    a.ado_per_tile = std::max(1, elems * kThreads / M);
+    a.tiles = (n_ado + a.ado_per_tile - 1) / a.ado_per_tile;
+    if ((int64_t)B * a.tiles >= 512) break;
+  }
   a.xcd_map = B >= kXcds;
   a.Hop = (const double2*)Hop;
   a.shift = shift;
@@ -657,7 +740,7 @@ static int heom_apply_impl(const qsx::HeomArgs& a, const void* y, void* out, voi
   const int ngroups = a.xcd_map ? kXcds * ((a.B + kXcds - 1) / kXcds) * a.tiles : a.B * a.tiles;
   HeomStageBufs<double> none{};
   hipLaunchKernelGGL(kern, dim3(ngroups), dim3(kThreads), shmem, as_stream(stream), a,
-                     (const double2*)y, (double2*)out, none, 0.0, 4);
+                     y, (double2*)out, none, 0.0, 4);
   QSX_CHECK_HIP(hipGetLastError());
   return QSX_OK;
 }
@@ -695,7 +778,7 @@ extern "C" int64_t qsx_heom_workspace_bytes(int32_t precision, int32_t B, int32_
                                             int32_t M) {
   if (B < 1 || n_ado < 1 || M < 1 || (precision != QSX_FP64 && precision != QSX_MIXED)) return -1;
   const int64_t total = (int64_t)B * n_ado * M;
-  return total * qsx::heom_bytes_per_element(precision == QSX_FP64);
+  return total * qsx::heom_bytes_per_element(precision == QSX_FP64, false);
 }
 
 static int heom_propagate_impl(int precision, const qsx::HeomArgs& a, const void* y0,
