@@ -1658,16 +1658,20 @@ extern "C" int32_t qsx_absorption_operators(const int64_t* table, int32_t B, int
                 "qsx_absorption_operators: flags %d (secular, real correlation, Heisenberg only)",
                 flags);
   const size_t lds = abs_lds_bytes(max_n);
-  // 256 threads per problem at every size: wider work-groups shorten a
-  // problem's Jacobi rounds but leave fewer compute units to the other
-  // size classes and the propagation running beside them
-  constexpr int kAbsThreads = 256;
+  // 256 threads per problem: wider work-groups shorten a problem's Jacobi
+  // rounds but leave fewer compute units to the other size classes and the
+  // propagation running beside them.  One wavefront up to eight sites, where a
+  // Jacobi round has at most 48 items: its barriers cost nothing and four times
+  // as many problems share the chip.  Few problems keep 256 threads for the
+  // summed Matsubara form of baths outside the closed form's range.
+  const auto kern = max_n <= 8 && B >= 64 ? absorption_ops_kernel<64> : absorption_ops_kernel<256>;
+  const int threads = max_n <= 8 && B >= 64 ? 64 : 256;
   if (lds > 64 * 1024)
-    QSX_CHECK_HIP(hipFuncSetAttribute((const void*)absorption_ops_kernel<kAbsThreads>,
+    QSX_CHECK_HIP(hipFuncSetAttribute((const void*)kern,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(absorption_ops_kernel<kAbsThreads>, dim3(B), dim3(kAbsThreads), lds,
-                     as_stream(stream), table, max_n, H1, rw, bath, flags, unit_convert, h, J,
-                     static_cast<double2*>(P1), static_cast<double2*>(PJ));
+  hipLaunchKernelGGL(kern, dim3(B), dim3(threads), lds, as_stream(stream), table, max_n, H1, rw,
+                     bath, flags, unit_convert, h, J, static_cast<double2*>(P1),
+                     static_cast<double2*>(PJ));
   QSX_CHECK_HIP(hipGetLastError());
   return QSX_OK;
 }
