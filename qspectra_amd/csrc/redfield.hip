@@ -32,6 +32,8 @@ namespace {
 
 constexpr int kMaxBlock = 64;  // Jacobi in LDS
 constexpr int kThreads = 256;
+constexpr int kWideBlock = 12;     // larger blocks: kWideThreads threads per record
+constexpr int kWideThreads = 512;
 
 __host__ __device__ inline int block_size(int X, int n) {
   return X == 0 ? 1 : (X == 1 ? n : n * (n - 1) / 2);
@@ -165,27 +167,38 @@ __device__ void jacobi_sweeps(double* A, double* V, int m, double (*rot)[2], int
   }
 }
 
-__global__ __launch_bounds__(kThreads) void block_eigh_kernel(const double* __restrict__ H1, int n,
-                                                              int X, const double* __restrict__ rw,
-                                                              const double* __restrict__ Hd,
-                                                              int nbd, double* __restrict__ ws,
-                                                              size_t rstride) {
-  __shared__ double A[kMaxBlock * kMaxBlock];
-  __shared__ double V[kMaxBlock * kMaxBlock];
+// One Hilbert block of a launch: its Hamiltonian (H, dense [B, nb, nb], or
+// block X of the one-exciton one), couplings (occ, diagonal over the block
+// basis, or block X's), bath table (or null: the Debye forms) and records.
+struct RecJob {
+  const double* H;
+  const double* occ;
+  const double2* ctab;
+  double* ws;
+  int X, nb;
+};
+
+// Eigenvalues and eigenvectors of problem b's block into its record.
+template <int NT>
+__device__ void block_eigh(const double* __restrict__ H1, int n, const double* __restrict__ rw,
+                           const RecJob& job, int b, const Rec& rec) {
+  extern __shared__ double rec_lds[];       // A and V
   __shared__ double rot[kMaxBlock / 2][2];
   __shared__ int pqs[kMaxBlock / 2][2];
   __shared__ int pi_[kMaxBlock], pj_[kMaxBlock];
-  __shared__ double red[2][kThreads];
+  __shared__ double red[2 * NT / 64];
   __shared__ int perm[kMaxBlock];
-  const int b = blockIdx.x, tid = threadIdx.x;
-  const int nb = Hd ? nbd : block_size(X, n);
+  const int tid = threadIdx.x, X = job.X, nb = job.nb;
   const int m = nb + (nb & 1);
+  double* A = rec_lds;
+  double* V = A + m * m;
+  const double* Hd = job.H;
   const double* H = Hd ? Hd + (size_t)b * nb * nb : H1 + (size_t)b * n * n;
   const double shift = Hd ? 0.0 : X * (rw ? rw[b] : 0.0);
   if (!Hd && X == 2)
-    for (int s = tid; s < nb; s += kThreads) pair_of(s, n, pi_[s], pj_[s]);
+    for (int s = tid; s < nb; s += NT) pair_of(s, n, pi_[s], pj_[s]);
   __syncthreads();
-  for (int e = tid; e < m * m; e += kThreads) {
+  for (int e = tid; e < m * m; e += NT) {
     const int r = e / m, c = e % m;
     double v = 0.0;
     if (r < nb && c < nb) {
@@ -204,10 +217,10 @@ __global__ __launch_bounds__(kThreads) void block_eigh_kernel(const double* __re
     V[e] = (r == c) ? 1.0 : 0.0;
   }
   __syncthreads();
-  jacobi_sweeps<kThreads>(A, V, m, rot, pqs, &red[0][0]);
+  jacobi_sweeps<NT>(A, V, m, rot, pqs, red);
   // ascending eigenvalues (stable ranking), canonical sign: the largest-
   // magnitude component of each eigenvector is made positive
-  for (int k = tid; k < nb; k += kThreads) {
+  for (int k = tid; k < nb; k += NT) {
     const double vk = A[k * m + k];
     int rank = 0;
     for (int l = 0; l < nb; ++l) {
@@ -217,8 +230,7 @@ __global__ __launch_bounds__(kThreads) void block_eigh_kernel(const double* __re
     perm[rank] = k;
   }
   __syncthreads();
-  Rec rec = rec_at(ws + (size_t)b * rstride, nb, n);
-  for (int k = tid; k < nb; k += kThreads) {
+  for (int k = tid; k < nb; k += NT) {
     const int c = perm[k];
     int best = 0;
     double bv = -1.0;
@@ -247,7 +259,10 @@ __device__ __forceinline__ double recip_nr(double d) {
   return r;
 }
 
-// The terms k = k0, k0 + stride, ... (< 1000) of the Matsubara sum: four
+// The terms k = k0, k0 + stride, ... (< 1000) of the Matsubara sum
+// sum_{k=1}^{999} nu_k / ((nu_k^2 - g^2)(nu_k - i x)), nu_k = 2 pi k T (its
+// value at -x is the complex conjugate, exactly so in floating point: only
+// signs change): four
 // interleaved Kahan-compensated sums (their reciprocals independent, so
 // they overlap), added at the end
 __device__ double2 matsubara_partial(double x, double T, double gam, int k0, int stride) {
@@ -272,14 +287,6 @@ __device__ double2 matsubara_partial(double x, double T, double gam, int k0, int
     }
   }
   return make_double2((sr[0] + sr[1]) + (sr[2] + sr[3]), (si[0] + si[1]) + (si[2] + si[3]));
-}
-
-// sum_{k=1}^{999} nu_k / ((nu_k^2 - g^2)(nu_k - i x)), nu_k = 2 pi k T,
-// compensated as above; its value at -x is the complex conjugate (each
-// term's imaginary part is odd in x, its real part even), exactly so in
-// floating point since only signs change
-__device__ double2 matsubara_sum(double x, double T, double gam) {
-  return matsubara_partial(x, T, gam, 1, 1);
 }
 
 // digamma of a complex argument away from the poles 0, -1, -2, ...: the
@@ -354,21 +361,24 @@ __device__ double2 debye_corr_with(double x, double2 S, double T, double lam, do
   return make_double2(lam * gam * re, lam * gam * im);
 }
 
-__global__ __launch_bounds__(kThreads) void block_bath_kernel(int n, int X, int nb,
-                                                              const double* __restrict__ occ,
-                                                              double T, double lam,
-                                                              double gam, int real_corr,
-                                                              double* __restrict__ ws,
-                                                              size_t rstride,
-                                                              const double2* __restrict__ ctab) {
-  const int b = blockIdx.x, tid = threadIdx.x;
-  Rec rec = rec_at(ws + (size_t)b * rstride, nb, n);
+// C(w) of every ordered pair of the block's eigenstates and the couplings K.
+// Each Matsubara sum (pairs d <= c: one sum serves C[d][c] and C[c][d]) is
+// 999 terms of a serial compensated chain: as many neighbouring lanes as the
+// work-group has for each pair share it, the partial sums added across them.
+template <int NT>
+__device__ void block_bath(int n, const RecJob& job, double T, double lam, double gam,
+                           int real_corr, int b, const Rec& rec) {
+  const int tid = threadIdx.x, X = job.X, nb = job.nb;
+  const double* __restrict__ occ = job.occ;
   // a tabulated bath: C[d][c] = C(E_d - E_c) given per problem
-  if (ctab != nullptr)
-    for (int e = tid; e < nb * nb; e += kThreads) rec.C[e] = ctab[(size_t)b * nb * nb + e];
-  // pairs (d, c) with d <= c: one Matsubara sum serves C[d][c] and C[c][d]
-  const int npairs = ctab != nullptr ? 0 : nb * (nb + 1) / 2;
-  for (int e = tid; e < npairs; e += kThreads) {
+  if (job.ctab != nullptr)
+    for (int e = tid; e < nb * nb; e += NT) rec.C[e] = job.ctab[(size_t)b * nb * nb + e];
+  const int npairs = job.ctab != nullptr ? 0 : nb * (nb + 1) / 2;
+  int S = 16;                       // lanes per pair
+  while (S > 1 && S * npairs > NT) S /= 2;
+  const int sub = tid & (S - 1);
+  for (int e0 = 0; e0 < npairs; e0 += NT / S) {          // uniform: the lanes of a pair add up
+    const int e = min(e0 + tid / S, npairs - 1);
     int d = 0, r = e;
     while (r >= nb - d) {
       r -= nb - d;
@@ -377,14 +387,19 @@ __global__ __launch_bounds__(kThreads) void block_bath_kernel(int n, int X, int 
     const int c = d + r;
     const double x = rec.E[d] - rec.E[c];
     const bool sum = !real_corr && x != 0.0;
-    const double2 S = sum ? matsubara_sum(x, T, gam) : make_double2(0.0, 0.0);
-    rec.C[d * nb + c] = debye_corr_with(x, S, T, lam, gam, real_corr);
-    if (c != d) rec.C[c * nb + d] = debye_corr_with(-x, make_double2(S.x, -S.y), T, lam, gam,
+    double2 M = sum ? matsubara_partial(x, T, gam, 1 + sub, S) : make_double2(0.0, 0.0);
+    for (int o = 1; o < S; o *= 2) {
+      M.x += __shfl_xor(M.x, o);
+      M.y += __shfl_xor(M.y, o);
+    }
+    if (sub != 0 || e0 + tid / S >= npairs) continue;
+    rec.C[d * nb + c] = debye_corr_with(x, M, T, lam, gam, real_corr);
+    if (c != d) rec.C[c * nb + d] = debye_corr_with(-x, make_double2(M.x, -M.y), T, lam, gam,
                                                     real_corr);
   }
   // K_i[a][m] = sum over states s of X that contain site i of U[s][a] U[s][m]
   const int nk = n * nb * nb;
-  for (int e = tid; e < nk; e += kThreads) {
+  for (int e = tid; e < nk; e += NT) {
     const int i = e / (nb * nb), a = (e / nb) % nb, m = e % nb;
     double v = 0.0;
     if (occ) {                       // diagonal coupling: occ[i][s] over the block basis
@@ -407,11 +422,10 @@ __global__ __launch_bounds__(kThreads) void block_bath_kernel(int n, int X, int 
 }
 
 // --------------------------------------------------------------------- 3. Gs
-__global__ __launch_bounds__(kThreads) void block_gs_kernel(int n, int nb, double* __restrict__ ws,
-                                                            size_t rstride) {
-  const int b = blockIdx.x, tid = threadIdx.x;
-  Rec rec = rec_at(ws + (size_t)b * rstride, nb, n);
-  for (int e = tid; e < nb * nb; e += kThreads) {
+template <int NT>
+__device__ void block_gs(int n, int nb, const Rec& rec) {
+  const int tid = threadIdx.x;
+  for (int e = tid; e < nb * nb; e += NT) {
     const int a = e / nb, c = e % nb;
     double2 g = make_double2(0.0, 0.0);
     for (int i = 0; i < n; ++i) {
@@ -425,6 +439,48 @@ __global__ __launch_bounds__(kThreads) void block_gs_kernel(int n, int nb, doubl
     }
     rec.Gs[e] = g;
   }
+}
+
+// A block's record in one pass: eigenstates, C and K, Gs.  grid (B, blocks): the
+// two blocks of a Liouvillian side by side in one launch, where six launches
+// one after the other left the chip to the smaller block's latency.  Wide
+// blocks take 512 threads (their rotations and pairs fill them; with 256 the
+// mean below took 1604 us for 1589, with 1024, whose barriers cost more, 1735).
+// Measured: the mean 2-D spectrum of 256 systems of 7 sites, whose blocks of 21
+// states bound it, 1763 -> 1544 us; the C gradient (below) of 512 systems of 7
+// sites, one lane per pair before, 140 -> 96 us.
+template <int NT>
+__global__ __launch_bounds__(NT) void block_rec_kernel(const double* __restrict__ H1, int n,
+                                                       const double* __restrict__ rw, double T,
+                                                       double lam, double gam, int real_corr,
+                                                       RecJob j0, RecJob j1, size_t rstride,
+                                                       int eig_only) {
+  const RecJob job = blockIdx.y ? j1 : j0;
+  const int b = blockIdx.x;
+  const Rec rec = rec_at(job.ws + (size_t)b * rstride, job.nb, n);
+  block_eigh<NT>(H1, n, rw, job, b, rec);
+  if (eig_only) return;
+  __syncthreads();
+  block_bath<NT>(n, job, T, lam, gam, real_corr, b, rec);
+  __syncthreads();
+  block_gs<NT>(n, job.nb, rec);
+}
+
+// The records of one or two blocks of B problems.
+void launch_recs(const double* H1, int n, int B, const double* rw, double T, double lam,
+                 double gam, int real_corr, const RecJob* jobs, int njobs, size_t rstride,
+                 int eig_only, hipStream_t s) {
+  const RecJob j1 = jobs[njobs - 1];
+  const int nb = std::max(jobs[0].nb, j1.nb), m = nb + (nb & 1);
+  const bool wide = nb > kWideBlock;
+  // sized by the blocks at hand: small ones fill a CU's threads, not its LDS
+  const size_t lds = 2 * (size_t)m * m * sizeof(double);
+  if (lds > 60 * 1024)
+    (void)hipFuncSetAttribute((const void*)block_rec_kernel<kWideThreads>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const auto kern = wide ? block_rec_kernel<kWideThreads> : block_rec_kernel<kThreads>;
+  hipLaunchKernelGGL(kern, dim3(B, njobs), dim3(wide ? kWideThreads : kThreads), lds, s, H1, n,
+                     rw, T, lam, gam, real_corr, jobs[0], j1, rstride, eig_only);
 }
 
 // sandwich: out[i + nX j] = sum_{a,b} UX[i][a] Z[a + nX b] UY[j][b]  (LDS)
@@ -971,9 +1027,11 @@ __global__ __launch_bounds__(NT) void absorption_ops_kernel(
 // Om = U^T Ubar (F = 0 where E_c = E_a); the f block's Hbar is gathered back
 // onto H1 through operator_1_to_2's four terms.
 
-// C(x)/lam and dC/dx of the Debye bath (the x = 0 branch is a constant)
+// C(x)/lam and dC/dx of the Debye bath (the x = 0 branch is a constant), by
+// S neighbouring lanes (a power of two, sub = 0 .. S - 1, the same x): each
+// takes every S-th term of the two sums
 __device__ void debye_corr_grad(double x, double T, double lam, double gam, int real_corr,
-                                double2& c1, double2& dc) {
+                                int sub, int S, double2& c1, double2& dc) {
   if (real_corr) {
     if (x == 0.0) {
       c1 = make_double2(T * 2.0 / gam, 0.0);
@@ -993,23 +1051,31 @@ __device__ void debye_corr_grad(double x, double T, double lam, double gam, int 
     dc = make_double2(0.0, 0.0);
     return;
   }
-  const double2 S = matsubara_sum(x, T, gam);
+  double2 M = matsubara_partial(x, T, gam, 1 + sub, S);
+  for (int o = 1; o < S; o *= 2) {
+    M.x += __shfl_xor(M.x, o);
+    M.y += __shfl_xor(M.y, o);
+  }
   const double ct = 1.0 / tan(gam / (2.0 * T));
   const double den = gam * gam + x * x;
-  c1 = make_double2(gam * ((ct * gam + x) / den + 4.0 * T * S.x),
-                    gam * ((ct * x - gam) / den + 4.0 * T * S.y));
+  c1 = make_double2(gam * ((ct * gam + x) / den + 4.0 * T * M.x),
+                    gam * ((ct * x - gam) / den + 4.0 * T * M.y));
   // d/dx (ct - i)/(g - i x) = (1 + i ct)(g^2 - x^2 + 2 i g x) / (g^2 + x^2)^2
   const double pr = gam * gam - x * x, pi = 2.0 * gam * x, d2 = den * den;
   double dr = (pr - ct * pi) / d2, di = (ct * pr + pi) / d2;
   // dS/dx = sum_k nu/(nu^2 - g^2) (-2 nu x + i (nu^2 - x^2)) / (nu^2 + x^2)^2
   double sr = 0.0, si = 0.0;
   const double twopiT = 2.0 * M_PI * T;
-  for (int k = 1; k < 1000; ++k) {
+  for (int k = 1 + sub; k < 1000; k += S) {
     const double nu = twopiT * k;
     const double q = nu * nu + x * x;
     const double f = nu / ((nu * nu - gam * gam) * q * q);
     sr = fma(f, -2.0 * nu * x, sr);
     si = fma(f, nu * nu - x * x, si);
+  }
+  for (int o = 1; o < S; o *= 2) {
+    sr += __shfl_xor(sr, o);
+    si += __shfl_xor(si, o);
   }
   dr += 4.0 * T * sr;
   di += 4.0 * T * si;
@@ -1236,9 +1302,15 @@ __global__ __launch_bounds__(kThreads) void vjp_chain_kernel(
     if (isy) g = cadd(g, GY[e]);
     Gsb[e] = g;
     Om[e] = (isx ? OX[e].x : 0.0) + (isy ? OY[e].x : 0.0);
-    const int d = e / nb, c = e % nb;
+  }
+  // the sums of a pair by as many neighbouring lanes as there are for each
+  int S = 16;
+  while (S > 1 && S * nb2 > kThreads) S /= 2;
+  for (int e0 = 0; e0 < nb2; e0 += kThreads / S) {
+    const int e = min(e0 + tid / S, nb2 - 1), d = e / nb, c = e % nb;
     double2 c1, dc;
-    debye_corr_grad(r.E[d] - r.E[c], T, lam, gam, real_corr, c1, dc);
+    debye_corr_grad(r.E[d] - r.E[c], T, lam, gam, real_corr, tid & (S - 1), S, c1, dc);
+    if ((tid & (S - 1)) != 0 || e0 + tid / S >= nb2) continue;
     C1[e] = c1;
     dC[e] = dc;
   }
@@ -1454,8 +1526,8 @@ extern "C" int32_t qsx_block_eigh(const double* H1, int32_t n, int32_t B, int32_
   const size_t rs = rec_doubles(nb, n);
   double* ws = static_cast<double*>(workspace);
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(block_eigh_kernel, dim3(B), dim3(kThreads), 0, s, H1, n, X, rw,
-                     (const double*)nullptr, 0, ws, rs);
+  const RecJob job = {nullptr, nullptr, nullptr, ws, X, nb};
+  launch_recs(H1, n, B, rw, 1.0, 0.0, 1.0, 0, &job, 1, rs, 1, s);
   QSX_CHECK_HIP(hipGetLastError());
   QSX_CHECK_HIP(hipMemcpy2DAsync(E, nb * sizeof(double), ws, rs * sizeof(double),
                                  nb * sizeof(double), B, hipMemcpyDeviceToDevice, s));
@@ -1505,19 +1577,9 @@ static int redfield_block_impl(const double* H1, int n, int B, const double* rw,
   double* wsX = static_cast<double*>(workspace);
   double* wsY = (X == Y) ? wsX : wsX + rs * B;
   double2* W = reinterpret_cast<double2*>(wsX + 2 * rs * B);
-  const int blocks[2] = {X, Y};
-  double* recs[2] = {wsX, wsY};
-  const double2* ctabs[2] = {static_cast<const double2*>(ctabX),
-                             static_cast<const double2*>(ctabY)};
-  for (int k = 0; k < (X == Y ? 1 : 2); ++k) {
-    const int nb = block_size(blocks[k], n);
-    hipLaunchKernelGGL(block_eigh_kernel, dim3(B), dim3(kThreads), 0, s, H1, n, blocks[k], rw,
-                       (const double*)nullptr, 0, recs[k], rs);
-    hipLaunchKernelGGL(block_bath_kernel, dim3(B), dim3(kThreads), 0, s, n, blocks[k], nb,
-                       (const double*)nullptr, T, lam, gam, (int)((flags & kRealCorr) != 0),
-                       recs[k], rs, ctabs[k]);
-    hipLaunchKernelGGL(block_gs_kernel, dim3(B), dim3(kThreads), 0, s, n, nb, recs[k], rs);
-  }
+  const RecJob jobs[2] = {{nullptr, nullptr, static_cast<const double2*>(ctabX), wsX, X, nX},
+                          {nullptr, nullptr, static_cast<const double2*>(ctabY), wsY, Y, nY}};
+  launch_recs(H1, n, B, rw, T, lam, gam, (flags & kRealCorr) != 0, jobs, X == Y ? 1 : 2, rs, 0, s);
   // non-secular blocks whose transformed factors fit the LDS: one pass
   const size_t kron = kron_lds_bytes(n, nX, nY);
   if (!(flags & kSecular) && n <= kKronMaxSites && kron <= 160 * 1024) {
@@ -1579,8 +1641,8 @@ extern "C" int32_t qsx_dense_eigh(const double* H, int32_t nb, int32_t B, double
   const size_t rs = rec_doubles(nb, 1);
   double* ws = static_cast<double*>(workspace);
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(block_eigh_kernel, dim3(B), dim3(kThreads), 0, s, (const double*)nullptr, 1,
-                     0, (const double*)nullptr, H, nb, ws, rs);
+  const RecJob job = {H, nullptr, nullptr, ws, 0, nb};
+  launch_recs(nullptr, 1, B, nullptr, 1.0, 0.0, 1.0, 0, &job, 1, rs, 1, s);
   QSX_CHECK_HIP(hipGetLastError());
   QSX_CHECK_HIP(hipMemcpy2DAsync(E, nb * sizeof(double), ws, rs * sizeof(double),
                                  nb * sizeof(double), B, hipMemcpyDeviceToDevice, s));
@@ -1609,18 +1671,9 @@ extern "C" int32_t qsx_redfield_block_dense(const double* HX, const double* HY, 
   double* wsY = same ? wsX : wsX + rs * B;
   double2* W = reinterpret_cast<double2*>(wsX + 2 * rs * B);
   hipStream_t s = as_stream(stream);
-  const double* Hs[2] = {HX, HY};
-  const double* occs[2] = {occX, occY};
-  const int nbs[2] = {nX, nY};
-  double* recs[2] = {wsX, wsY};
-  for (int k = 0; k < (same ? 1 : 2); ++k) {
-    hipLaunchKernelGGL(block_eigh_kernel, dim3(B), dim3(kThreads), 0, s, (const double*)nullptr,
-                       n, 0, (const double*)nullptr, Hs[k], nbs[k], recs[k], rs);
-    hipLaunchKernelGGL(block_bath_kernel, dim3(B), dim3(kThreads), 0, s, n, 0, nbs[k], occs[k],
-                       T, lam, gam, (int)((flags & kRealCorr) != 0), recs[k], rs,
-                       (const double2*)nullptr);
-    hipLaunchKernelGGL(block_gs_kernel, dim3(B), dim3(kThreads), 0, s, n, nbs[k], recs[k], rs);
-  }
+  const RecJob jobs[2] = {{HX, occX, nullptr, wsX, 0, nX}, {HY, occY, nullptr, wsY, 0, nY}};
+  launch_recs(nullptr, n, B, nullptr, T, lam, gam, (flags & kRealCorr) != 0, jobs, same ? 1 : 2, rs,
+              0, s);
   const size_t shmem = 3 * (size_t)M * sizeof(double2) + (size_t)(nX * nX + nY * nY) * sizeof(double);
   QSX_CHECK_ARG(shmem <= 64 * 1024, "qsx_redfield_block_dense: block too large (M=%d)", M);
   hipLaunchKernelGGL(liouv_cols_kernel, dim3(M, B), dim3(kThreads), shmem, s, n, nX, nY,
@@ -1717,17 +1770,9 @@ extern "C" int32_t qsx_redfield_block_vjp(const double* H1, int32_t n, int32_t B
   const size_t rcount = vjp_red_count(n, nX, nY);
   double* chain = reinterpret_cast<double*>(red + rcount * B);
   const size_t cstride = vjp_slab_doubles(std::max(nX, nY));
-  const int blocks[2] = {X, Y};
-  double* recs[2] = {wsX, wsY};
-  for (int k = 0; k < (same ? 1 : 2); ++k) {
-    const int nb = block_size(blocks[k], n);
-    hipLaunchKernelGGL(block_eigh_kernel, dim3(B), dim3(kThreads), 0, s, H1, n, blocks[k], rw,
-                       (const double*)nullptr, 0, recs[k], rs);
-    hipLaunchKernelGGL(block_bath_kernel, dim3(B), dim3(kThreads), 0, s, n, blocks[k], nb,
-                       (const double*)nullptr, T, lam, gam, (int)((flags & kRealCorr) != 0),
-                       recs[k], rs, (const double2*)nullptr);
-    hipLaunchKernelGGL(block_gs_kernel, dim3(B), dim3(kThreads), 0, s, n, nb, recs[k], rs);
-  }
+  const RecJob jobs[2] = {{nullptr, nullptr, nullptr, wsX, X, nX},
+                          {nullptr, nullptr, nullptr, wsY, Y, nY}};
+  launch_recs(H1, n, B, rw, T, lam, gam, (flags & kRealCorr) != 0, jobs, same ? 1 : 2, rs, 0, s);
   const double2* G = static_cast<const double2*>(gL);
   if (!(flags & kEigenBasis)) {
     hipLaunchKernelGGL(vjp_cols_kernel, dim3(M, B), dim3(kThreads), shmem, s, n, nX, nY, wsX,

@@ -308,3 +308,28 @@ def test_redfield_vjp_matches_finite_differences(gpu, X, Y, secular, heis, eigen
         assert np.all(np.abs(fd - an) <= 1e-6 * scale), (p, q, fd, an)
     fdl = (loss(H, BATH[1] + 1e-4) - loss(H, BATH[1] - 1e-4)) / 2e-4
     assert np.all(np.abs(fdl - glam) <= 1e-6 * np.abs(fdl)), (fdl, glam)
+
+
+@pytest.mark.parametrize('n', [1, 2, 12, 13, 17, 33])
+def test_records_across_widths(gpu, n):
+    """Block records over the lanes per Matsubara sum (16 down to 1, pairs
+    in several trips) and both work-group widths (the line lies at 12
+    states): block eg and its cotangents against the torch restatement, with
+    the bounds of the comparison above."""
+    from tests import torch_redfield as TR
+    H = _sym_h(n, 2, n)
+    rw = np.array([12450.0, 12380.0])
+    rng = np.random.RandomState(n)
+    Hd, rwd = torch.as_tensor(H).cuda(), torch.as_tensor(rw).cuda()
+    L = _native.redfield_block(Hd, rwd, *BATH, 1, 0, 0, S.CM_FS)
+    gL = torch.as_tensor(_cplx(rng, *L.shape)).cuda()
+    gH, glam = _native.redfield_block_vjp(Hd, rwd, *BATH, 1, 0, 0, S.CM_FS, gL)
+    for b in range(2):
+        Ht = torch.tensor(H[b:b + 1], requires_grad=True)
+        lam = torch.tensor(BATH[1], dtype=torch.float64, requires_grad=True)
+        Lt = TR.redfield_block(Ht, lam, BATH[2], BATH[0], rw[b], 'e', 'g', False, False, S.CM_FS)
+        assert rel_err(L[b].cpu().numpy(), Lt[0].detach().numpy()) < 1e-12
+        (torch.conj(gL[b:b + 1].cpu()) * Lt).real.sum().backward()
+        ref = (Ht.grad[0] + Ht.grad[0].T).numpy() / 2
+        assert np.abs(gH[b].cpu().numpy() - ref).max() < 1e-9 * np.abs(ref).max()
+        assert abs(float(glam[b]) - float(lam.grad)) < 1e-9 * abs(float(lam.grad))
