@@ -634,6 +634,13 @@ int64_t qsx_fourier_workspace_bytes(int32_t N);
 int32_t qsx_fourier_transform(const void* x, int64_t batch, int32_t n, int32_t N, int32_t lo,
                               int32_t sign, double dt, int32_t adjoint, void* workspace,
                               void* out, void* stream);
+/* The real part of qsx_fourier_transform (adjoint = 0): out [batch][N] float64.
+ * For the sizes where qsx_fourier_real_pairs is 1 (long rows whose samples
+ * start at the grid's zero); workspace as above. */
+int32_t qsx_fourier_real_pairs(int32_t n, int32_t N, int32_t lo);
+int32_t qsx_fourier_transform_real(const void* x, int64_t batch, int32_t n, int32_t N,
+                                   int32_t lo, int32_t sign, double dt, void* workspace,
+                                   double* out, void* stream);
 
 #ifdef __cplusplus
 }

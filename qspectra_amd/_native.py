@@ -116,6 +116,9 @@ SIGNATURES = {
     'qsx_fourier_workspace_bytes': [c_i32],
     'qsx_fourier_transform': [c_vp, c_i64, c_i32, c_i32, c_i32, c_i32, ctypes.c_double, c_i32,
                               c_vp, c_vp, c_vp],
+    'qsx_fourier_real_pairs': [c_i32, c_i32, c_i32],
+    'qsx_fourier_transform_real': [c_vp, c_i64, c_i32, c_i32, c_i32, c_i32, ctypes.c_double,
+                                   c_vp, c_vp, c_vp],
     'qsx_propagator_workspace_bytes': [c_i32, c_i32],
     'qsx_rk4_propagator': [c_vp, c_i64, c_i32, c_i32, c_dbl, c_i32, c_vp, c_vp, c_i64, c_vp],
     'qsx_rk4_propagator_noalloc': [c_vp, c_i64, c_i32, c_i32, c_dbl, c_i32, c_vp, c_vp],
@@ -1197,6 +1200,24 @@ def fourier_transform(x, N, lo, sign, dt, stream=None):
     """qsx_fourier_transform along the last axis of a device tensor:
     [..., n] samples -> [..., N] on the zero-padded symmetric grid."""
     return _fourier(x, x.shape[-1], N, lo, sign, dt, False, stream)
+
+
+def fourier_transform_real(x, N, lo, sign, dt, stream=None):
+    """The real part of fourier_transform: float64 [..., N] (two rows per
+    transform where qsx_fourier_real_pairs takes the sizes)."""
+    lib = require_native()
+    n, lead = x.shape[-1], tuple(x.shape[:-1])
+    batch = int(np.prod(lead)) if lead else 1
+    if batch < 2 or not lib.qsx_fourier_real_pairs(int(n), int(N), int(lo)):
+        return fourier_transform(x, N, lo, sign, dt, stream).real
+    x = x.to(torch.complex128).contiguous()
+    out = torch.empty(lead + (N,), dtype=torch.float64, device=x.device)
+    nbytes = lib.qsx_fourier_workspace_bytes(int(N))
+    ws = torch.empty((nbytes + 15) // 16, dtype=torch.complex128, device=x.device)
+    check(lib.qsx_fourier_transform_real(ptr(x), batch, int(n), int(N), int(lo), int(sign),
+                                         float(dt), ptr(ws), ptr(out), stream_ptr(stream)),
+          'qsx_fourier_transform_real')
+    return out
 
 
 def fourier_transform_adjoint(g, n, lo, sign, dt, stream=None):

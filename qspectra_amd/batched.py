@@ -43,8 +43,8 @@ def absorption_batch(hamiltonians, time_max, rw_freq, dt, model_cls=RedfieldMode
         x = torch.as_tensor(signal).to(_native.device())
         if correlation_decay_time is not None:
             x = x * torch.as_tensor(np.exp(-ticks / correlation_decay_time)).to(x.device)
-        f, X = fourier_transform_device(ticks, -x, -1, rw_freq, unit_convert)
-        X = X.real.cpu().numpy()
+        f, X = fourier_transform_device(ticks, -x, -1, rw_freq, unit_convert, real=True)
+        X = X.cpu().numpy()
         if out is None:
             out = np.empty((len(hamiltonians), X.shape[-1]))
         out[idx] = X
@@ -295,9 +295,9 @@ class AbsorptionEnsemblePlan(object):
         # the transform's scale
         x = self.signal if self.decay is None else self.signal * self._decay
         f, X = fourier_transform_device(self.t, x, -1, self.rw_freq, self.unit_convert,
-                                        scale=-1.0)
+                                        scale=-1.0, real=True)
         self.f = f
-        return X.real
+        return X
 
     def capture(self):
         """Records the whole plan into one HIP graph, replayed by run()."""

@@ -502,6 +502,160 @@ __global__ __launch_bounds__(kFftThreads) void chirp_rows_kernel(
   }
 }
 
+// The real parts of two rows' transforms at once, where the samples start at
+// the grid's zero (v + D = v >= 0): Re X[u] is the transform of the row's
+// Hermitian extension (x[v] / 2 at v > 0, conj(x[v]) / 2 at -v, Re x[0]), so
+// one complex transform of h_a + i h_b has the two real parts as its real and
+// imaginary part.  Both halves of the extension are pieces of n samples; a
+// chunk's spectrum is the sum of their products, so a pair of rows takes two
+// forward FFTs and one inverse FFT per chunk, where two rows alone take two
+// forward and two inverse FFTs per chunk, and the output is written as
+// doubles.  Row b is scaled by a power of two to row a's magnitude (each
+// row's rounding error stays relative to its own); rows that cannot share
+// (non-finite, zero, or beyond the exponent range) are transformed one by one:
+// row a in the first launch, which marks row b for the second (ALONE).
+// MEASURED
+constexpr long long kAloneMark = 0x7ff8000000a10e5eLL;   // a NaN
+
+template <bool ALONE>
+__global__ __launch_bounds__(kFftThreads) void chirp_pairs_kernel(
+    const double2* __restrict__ in, int64_t batch, ChirpGeom g, const double2* __restrict__ cin,
+    const double2* __restrict__ cout, const double2* __restrict__ Gt, double scale,
+    double* __restrict__ out) {
+  extern __shared__ double2 lds[];
+  double2* buf = lds;
+  double2* tw1 = lds + kFftPadded;
+  double2* tw2 = tw1 + kTw1;
+  __shared__ double smax[2][kFftThreads / 64];
+  const int t = threadIdx.x, n = g.P;
+  const double oscale = scale / (double)kFftL;
+  const int64_t ra = 2 * (int64_t)blockIdx.x, rb = ra + 1;
+  // the rows left alone by the first launch: their first entry holds the mark
+  if (ALONE && (rb >= batch || __double_as_longlong(out[rb * g.n_out]) != kAloneMark)) return;
+  build_fft_twiddles(tw1, tw2);
+  const double2* rowa = in + ra * n;
+  const double2* rowb = rb < batch ? in + rb * n : rowa;
+  int shift = 0, share = 0;
+  if (!ALONE) {
+    double ma = 0.0, mb = 0.0;
+    bool finite = true;
+#pragma unroll
+    for (int r = 0; r < kFftPer / 2; ++r) {
+      const int v = t + r * kFftThreads;
+      if (v < n) {
+        const double2 xa = rowa[v], xb = rowb[v];
+        finite = finite && isfinite(xa.x) && isfinite(xa.y) && isfinite(xb.x) && isfinite(xb.y);
+        ma = fmax(ma, fmax(fabs(xa.x), fabs(xa.y)));
+        mb = fmax(mb, fmax(fabs(xb.x), fabs(xb.y)));
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      ma = fmax(ma, __shfl_xor(ma, o));
+      mb = fmax(mb, __shfl_xor(mb, o));
+    }
+    if ((t & 63) == 0) {
+      smax[0][t >> 6] = ma;
+      smax[1][t >> 6] = mb;
+    }
+    const bool all_finite = __syncthreads_and(finite) != 0;
+    for (int q = 0; q < kFftThreads / 64; ++q) {
+      ma = fmax(ma, smax[0][q]);
+      mb = fmax(mb, smax[1][q]);
+    }
+    shift = __builtin_amdgcn_readfirstlane(ma > 0.0 && mb > 0.0 ? ilogb(ma) - ilogb(mb) : 0);
+    share = __builtin_amdgcn_readfirstlane(rb < batch && all_finite && ma > 0.0 && mb > 0.0 &&
+                                           abs(shift) < 500);
+  }
+  // the power of two of each row (0: not in it)
+  const double fa = ALONE ? 0.0 : 0.5, fb = ALONE ? 0.5 : (share ? ldexp(0.5, shift) : 0.0);
+  const double oa = oscale, ob = share ? ldexp(oscale, -shift) : oscale;
+  double2 S[kFftPer], R[kFftPer];
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half) {     // samples at v >= 0, then at v < 0
+    __syncthreads();
+#pragma unroll
+    for (int r0 = 0; r0 < kFftPer / 2; r0 += 4) {
+      double2 xa[4], xb[4], c[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int v = t + (r0 + q) * kFftThreads;
+        const int m = half == 0 ? v : n - v;            // the sample behind entry v
+        xa[q] = xb[q] = c[q] = make_double2(0.0, 0.0);
+        if (v < n && m < n) {
+          if (fa != 0.0) xa[q] = rowa[m];
+          if (fb != 0.0) xb[q] = rowb[m];
+          c[q] = cin[m];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int v = t + (r0 + q) * kFftThreads;
+        // h_a + i h_b
+        const double sg = half == 0 ? 1.0 : -1.0;
+        double2 w = make_double2(fa * xa[q].x - sg * (fb * xb[q].y),
+                                 sg * (fa * xa[q].y) + fb * xb[q].x);
+        if (half == 0 && v == 0) w = make_double2(2.0 * fa * xa[q].x, 2.0 * fb * xb[q].x);
+        const double2 y = cmul(w, c[q]);
+        buf[fpad(2 * v)] = y;
+        buf[fpad(2 * v + 1)] = y;
+      }
+    }
+    __syncthreads();
+    fft_tail_to_registers(buf, tw1, tw2, R);
+    if (half == 0)
+#pragma unroll
+      for (int r = 0; r < kFftPer; ++r) S[r] = R[r];
+  }
+  __syncthreads();                 // every thread's reads of buf are done
+  // chunk 0's spectrum through the radix-2 pass of its inverse FFT into
+  // LDS, chunk 1's kept in S (tables: chunk, then half v < 0, v >= 0)
+#pragma unroll
+  for (int q = 0; q < kFftPer / 2; ++q) {
+    const int jj = t + q * kFftThreads;
+    double2 e[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const double2* G = Gt + jj + u * (kFftL / 2);
+      const int x = q + u * (kFftPer / 2);
+      e[u] = cconj(cadd(cmul(S[x], G[kFftL]), cmul(R[x], G[0])));
+      if (g.chunks == 2)
+        S[x] = cconj(cadd(cmul(S[x], G[3 * kFftL]), cmul(R[x], G[2 * kFftL])));
+    }
+    buf[fpad(2 * jj)] = cadd(e[0], e[1]);
+    buf[fpad(2 * jj + 1)] = csub(e[0], e[1]);
+  }
+  for (int j = 0; j < g.chunks; ++j) {
+    const int j0 = j * g.H, he = min(g.H, g.n_out - j0);
+    if (j > 0) {
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kFftPer / 2; ++q) {
+        const int jj = t + q * kFftThreads;
+        buf[fpad(2 * jj)] = cadd(S[q], S[q + kFftPer / 2]);
+        buf[fpad(2 * jj + 1)] = csub(S[q], S[q + kFftPer / 2]);
+      }
+    }
+    __syncthreads();
+    {
+      double2 y[kFftPer];
+      fft_tail_to_registers(buf, tw1, tw2, y);
+#pragma unroll
+      for (int r = 0; r < kFftPer; ++r) buf[fpad(t + r * kFftThreads)] = y[r];
+    }
+#pragma unroll
+    for (int r = 0; r < kFftPer; ++r) {
+      const int u = t + r * kFftThreads;
+      if (u < he) {
+        const double2 z = cmul(cout[j0 + u], cconj(buf[fpad(u)]));
+        if (fa != 0.0) out[ra * g.n_out + j0 + u] = oa * z.x;
+        if (fb != 0.0) out[rb * g.n_out + j0 + u] = ob * z.y;
+      }
+    }
+  }
+  if (!ALONE && !share && rb < batch && t == 0)
+    out[rb * g.n_out] = __longlong_as_double(kAloneMark);
+}
+
 // Piece/chunk geometry of a transform, or false for the direct sum.
 bool chirp_geometry(int n_in, int n_out, int N, int64_t a0, int da, int64_t d0, int dd, int adj,
                     ChirpGeom* g) {
@@ -521,13 +675,19 @@ bool chirp_geometry(int n_in, int n_out, int N, int64_t a0, int da, int64_t d0, 
   return true;
 }
 
+// Whether chirp_pairs_kernel takes n samples at lo of N points: chirp lengths,
+// one piece, the first sample at the grid's zero, two chunks at most.
+bool chirp_pairs_ok(int n, int N, int lo) {
+  return n >= kChirpMin && n <= kFftL / 2 && lo == N / 2 && N <= 2 * (kFftL - n + 1);
+}
+
 // Entries (complex) of the chirp tables' workspace beyond the direct sum's
 // N-entry twiddle table: the input and output chirps (n_in + n_out <= 2N)
-// and the pair spectra.
+// and the pair spectra (four for the two halves and chunks of paired rows).
 int64_t chirp_workspace_entries(int64_t N) {
   if (N < kChirpMin) return 0;
   const int64_t per = (N + kFftL / 2 - 1) / (kFftL / 2);   // pieces or chunks, at most
-  return 2 * N + std::min<int64_t>(kChirpMaxTables, per * per) * kFftL;
+  return 2 * N + std::min<int64_t>(kChirpMaxTables, std::max<int64_t>(4, per * per)) * kFftL;
 }
 
 }  // namespace
@@ -588,6 +748,53 @@ extern "C" int32_t qsx_fourier_transform(const void* x, int64_t batch, int32_t n
   hipLaunchKernelGGL(kern, dim3((unsigned)gx, gy), dim3(kDftThreads), 0, s,
                      static_cast<const double2*>(x), batch, n_in, n_out, N, a0, da, d0, dd,
                      (int)(adjoint != 0), dt, T, static_cast<double2*>(out));
+  QSX_CHECK_HIP(hipGetLastError());
+  return QSX_OK;
+}
+
+extern "C" int32_t qsx_fourier_real_pairs(int32_t n, int32_t N, int32_t lo) {
+  return n >= 1 && N >= n && lo >= 0 && lo <= N - n && chirp_pairs_ok(n, N, lo) ? 1 : 0;
+}
+
+extern "C" int32_t qsx_fourier_transform_real(const void* x, int64_t batch, int32_t n, int32_t N,
+                                              int32_t lo, int32_t sign, double dt,
+                                              void* workspace, double* out, void* stream) {
+  QSX_CHECK_ARG(x && out && workspace, "qsx_fourier_transform_real: null pointer");
+  QSX_CHECK_ARG(batch >= 1 && batch < (int64_t)1 << 31 && qsx_fourier_real_pairs(n, N, lo),
+                "qsx_fourier_transform_real: bad sizes n=%d N=%d lo=%d batch=%lld", n, N, lo,
+                (long long)batch);
+  QSX_CHECK_ARG(sign == 1 || sign == -1, "qsx_fourier_transform_real: sign must be +1 or -1");
+  hipStream_t s = as_stream(stream);
+  double2* cin = static_cast<double2*>(workspace) + N;
+  double2* cout = cin + n;
+  double2* Gt = cin + 2 * (int64_t)N;
+  // output index r -> s_r = a0 + da r as in the complex transform; D = 0
+  const int64_t c = N / 2, a0 = sign == -1 ? -c : (int64_t)N - 1 - c;
+  const int da = sign == -1 ? 1 : -1;
+  ChirpGeom g;
+  g.n_in = n;
+  g.n_out = N;
+  g.P = n;
+  g.H = kFftL - n + 1;
+  g.pieces = 2;
+  g.chunks = (N + g.H - 1) / g.H;
+  g.sigma = da;
+  g.N = N;
+  g.A = da * a0;
+  g.D = 0;
+  hipLaunchKernelGGL(chirp_vectors_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, g,
+                     cin, cout);
+  g.D = -n;                          // the tables' pieces: v = -n .. -1, then 0 .. n - 1
+  QSX_CHECK_HIP(hipFuncSetAttribute((const void*)chirp_tables_kernel,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFftLds));
+  for (const void* k : {(const void*)chirp_pairs_kernel<false>, (const void*)chirp_pairs_kernel<true>})
+    QSX_CHECK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFftLds));
+  hipLaunchKernelGGL(chirp_tables_kernel, dim3(2 * g.chunks), dim3(kFftThreads), kFftLds, s, g,
+                     Gt);
+  for (const auto k : {chirp_pairs_kernel<false>, chirp_pairs_kernel<true>})
+    hipLaunchKernelGGL(k, dim3((unsigned)((batch + 1) / 2)), dim3(kFftThreads), kFftLds, s,
+                       static_cast<const double2*>(x), batch, g, (const double2*)cin,
+                       (const double2*)cout, (const double2*)Gt, dt, out);
   QSX_CHECK_HIP(hipGetLastError());
   return QSX_OK;
 }

@@ -462,12 +462,13 @@ class _SymmetricFourier(torch.autograd.Function):
 
 
 def fourier_transform_device(t, x, axis=-1, rw_freq=0, unit_convert=1, sign=1,
-                             convention='angular', scale=1.0):
+                             convention='angular', scale=1.0, real=False):
     """fourier_transform on a complex128 device tensor x (result stays on the
     device; differentiable): the zero-padded symmetric grid, ifftshift, DFT,
     fftshift of utils.py:128-219, evaluated by qsx_fourier_transform (a
     direct sum for short rows, the chirp-z form with FFTs in LDS for long
-    ones), the result times ``scale``."""
+    ones), the result times ``scale``.  With ``real`` its real part only (not
+    differentiable)."""
     t = np.asarray(t, dtype=float)
     if t.ndim != 1:
         raise ValueError('t must be one dimensional')
@@ -485,7 +486,11 @@ def fourier_transform_device(t, x, axis=-1, rw_freq=0, unit_convert=1, sign=1,
     N = t_sym.size
     dt = t_sym[1] - t_sym[0]
     xm = x.to(torch.complex128).movedim(ax, -1)
-    X = _SymmetricFourier.apply(xm, N, lo, sign, float(dt) * float(scale)).movedim(-1, ax)
+    factor = float(dt) * float(scale)
+    if real:
+        X = _native.fourier_transform_real(xm.detach(), N, lo, sign, factor).movedim(-1, ax)
+    else:
+        X = _SymmetricFourier.apply(xm, N, lo, sign, factor).movedim(-1, ax)
     f = np.fft.fftshift(np.fft.fftfreq(N, dt * unit_convert))
     if sign == 1:
         f = -f[::-1]

@@ -120,3 +120,29 @@ def test_direct_sum_row_groups(gpu, rows, n, lo, N):
         back = _native.fourier_transform_adjoint(g, n, lo, sign, 0.5)
         want = want @ F.conj()
         assert np.abs(back.cpu().numpy() - want).max() <= 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize('rows,n,sign', [(2, 2048, -1), (3, 2049, 1), (4, 3000, -1),
+                                         (5, 4096, 1), (2, 4095, -1)])
+def test_paired_real_parts(gpu, rows, n, sign):
+    """Real parts of two rows per transform against the complex transform:
+    one and two chunks, odd batches, rows of very different magnitude, a zero
+    and a non-finite row beside a finite one.  The rounding of log2(8192) = 13
+    passes each way, some tens of ulp: 1e-13 of the row's own scale."""
+    rs = np.random.RandomState(n)
+    N, lo = 2 * n - 1, n - 1
+    x = rs.normal(size=(rows, n)) + 1j * rs.normal(size=(rows, n))
+    x[1] *= 1e-12
+    if rows > 2:
+        x[2] = 0
+    if rows > 4:
+        x[2, 7] = np.nan
+    xd = torch.as_tensor(x).to('cuda')
+    want = _native.fourier_transform(xd, N, lo, sign, 0.5).real.cpu().numpy()
+    got = _native.fourier_transform_real(xd, N, lo, sign, 0.5).cpu().numpy()
+    assert got.dtype == np.float64 and got.shape == (rows, N)
+    for b in range(rows):
+        if np.isnan(x[b]).any():
+            assert np.isnan(got[b]).all()
+        else:
+            assert np.abs(got[b] - want[b]).max() <= 1e-13 * np.abs(want[b]).max()
