@@ -45,6 +45,22 @@ constexpr int kMaxStates = 31;  // rows M plus J projection rows in 64 lanes
 constexpr int kFlush = 32;      // signal values staged in LDS between stores
 constexpr int kMaxJ = 8;
 
+// The values staged up to step last, of count groups, out to their rows in
+// whole lines; a value that is not finite marks its group.
+__device__ __forceinline__ void flush_signals(int last, int count, int nt,
+                                              double2 (*sbuf)[kWave / 2], const int64_t* rows,
+                                              int* sbad, double2* __restrict__ out) {
+  const int k0 = last - last % kFlush, cnt = last - k0 + 1;
+  for (int e = threadIdx.x; e < count * kFlush; e += kWave) {
+    const int gi = e / kFlush, t = e % kFlush;
+    if (t < cnt) {
+      const double2 s = sbuf[t][gi];
+      out[rows[gi] * nt + k0 + t] = s;
+      if (!isfinite(s.x) || !isfinite(s.y)) sbad[gi] = 1;
+    }
+  }
+}
+
 // One wavefront's problems of M states through all nt steps, J per round
 // trip.  M is a template parameter so that the row product is straight-line
 // code: the M LDS reads of a round trip issue together before its
@@ -56,7 +72,7 @@ __device__ void bucket_wave(const int4 w, const int64_t* __restrict__ offs,
                             const double2* __restrict__ P, const double2* __restrict__ y0,
                             const double2* __restrict__ W, int nt, double2* __restrict__ out,
                             int32_t* __restrict__ status, double2 (*ys)[kWave],
-                            double2 (*sbuf)[kWave / 2], int64_t* rows, int (*sbad)[kMaxJ]) {
+                            double2 (*sbuf)[kWave / 2], int64_t* rows, int* sbad) {
   constexpr int kCols = (M + S - 1) / S;                 // columns per lane
   const int lane = threadIdx.x, G = w.w;
   const int g = lane / G, li = lane - g * G;
@@ -87,10 +103,12 @@ __device__ void bucket_wave(const int4 w, const int64_t* __restrict__ offs,
   }
   const int base = g * G;
   if (lead) ys[0][base + i] = srow ? y0[offY + i] : make_double2(0.0, 0.0);
-  if (live && li == 0) rows[g] = orow;   // for the coalesced flushes
+  if (live && li == 0) {                 // for the coalesced flushes
+    rows[g] = orow;
+    sbad[g] = 0;
+  }
   __syncthreads();
   const int nr = (nt + J - 1) / J;
-  bool bad = false;
   int cur = 0;
   for (int k = 0; k < nr; ++k) {
     double2 acc[4];
@@ -123,48 +141,24 @@ __device__ void bucket_wave(const int4 w, const int64_t* __restrict__ offs,
       sum.y += __shfl_xor(sum.y, 1);
     }
     const int step = k * J + jj;
-    if (prow && lead && step < nt) {
-      sbuf[step % kFlush][g] = sum;
-      bad |= !isfinite(sum.x) || !isfinite(sum.y);
-    }
+    if (prow && lead && step < nt) sbuf[step % kFlush][g] = sum;
     if (lead) ys[cur ^ 1][base + i] = sum;
     __syncthreads();
     cur ^= 1;
     const int last = min((k + 1) * J, nt) - 1;           // last step of this round trip
     if (last % kFlush == kFlush - 1 || k == nr - 1) {    // uniform: flush the staged values
-      const int k0 = last - last % kFlush, cnt = last - k0 + 1;
-      for (int e = lane; e < w.y * cnt; e += kWave) {
-        const int gi = e / cnt, t = e - gi * cnt;
-        out[rows[gi] * nt + k0 + t] = sbuf[t][gi];
-      }
+      flush_signals(last, w.y, nt, sbuf, rows, sbad, out);
       __syncthreads();
     }
   }
-  if (prow && lead) sbad[g][jj] = bad ? 1 : 0;
-  __syncthreads();
-  if (prow && lead && jj == 0) {
-    int any = 0;
-#pragma unroll
-    for (int j = 0; j < J; ++j) any |= sbad[g][j];
-    status[orow] = any;
-  }
-}
-
-// Entry N of a 16-lane row of v, broadcast to the row (DPP row_newbcast;
-// two 32-bit moves per double).
-template <int N>
-__device__ __forceinline__ double row_bcast(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0x150 + N, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x150 + N, 0xF, 0xF, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+  if (prow && lead && jj == 0) status[orow] = sbad[g];
 }
 
 // acc[j & 3] += row[j] y_j for j = Q .. M - 1, y_j held by lane j of the row
 template <int Q, int M>
 struct RowDot {
   static __device__ __forceinline__ void run(const double2* row, double2 y, double2* acc) {
-    const double2 yj = make_double2(row_bcast<Q>(y.x), row_bcast<Q>(y.y));
+    const double2 yj = make_double2(row_lane<Q>(y.x), row_lane<Q>(y.y));
     double2& a = acc[Q & 3];
     a.x = fma(row[Q].x, yj.x, a.x);
     a.x = fma(-row[Q].y, yj.y, a.x);
@@ -187,7 +181,7 @@ __device__ void bucket_wave_row(const int4 w, const int64_t* __restrict__ offs,
                                 const double2* __restrict__ P, const double2* __restrict__ y0,
                                 const double2* __restrict__ W, int nt, double2* __restrict__ out,
                                 int32_t* __restrict__ status, double2 (*sbuf)[kWave / 2],
-                                int64_t* rows, int (*sbad)[kMaxJ]) {
+                                int64_t* rows, int* sbad) {
   static_assert(M + J <= 16, "one problem per 16-lane row");
   const int lane = threadIdx.x;
   const int g = lane >> 4, i = lane & 15;
@@ -210,10 +204,12 @@ __device__ void bucket_wave_row(const int4 w, const int64_t* __restrict__ offs,
     row[j] = r;
   }
   double2 y = srow ? y0[offY + i] : make_double2(0.0, 0.0);
-  if (live && i == 0) rows[g] = orow;
+  if (live && i == 0) {
+    rows[g] = orow;
+    sbad[g] = 0;
+  }
   __syncthreads();
   const int nr = (nt + J - 1) / J;
-  bool bad = false;
   for (int k = 0; k < nr; ++k) {
     double2 acc[4];
 #pragma unroll
@@ -222,30 +218,16 @@ __device__ void bucket_wave_row(const int4 w, const int64_t* __restrict__ offs,
     const double2 sum = make_double2((acc[0].x + acc[1].x) + (acc[2].x + acc[3].x),
                                      (acc[0].y + acc[1].y) + (acc[2].y + acc[3].y));
     const int step = k * J + jj;
-    if (prow && step < nt) {
-      sbuf[step % kFlush][g] = sum;
-      bad |= !isfinite(sum.x) || !isfinite(sum.y);
-    }
+    if (prow && step < nt) sbuf[step % kFlush][g] = sum;
     y = sum;            // projection lanes' values are never broadcast
     const int last = min((k + 1) * J, nt) - 1;
     if (last % kFlush == kFlush - 1 || k == nr - 1) {    // uniform: flush the staged values
       __syncthreads();
-      const int k0 = last - last % kFlush, cnt = last - k0 + 1;
-      for (int e = lane; e < w.y * cnt; e += kWave) {
-        const int gi = e / cnt, t = e - gi * cnt;
-        out[rows[gi] * nt + k0 + t] = sbuf[t][gi];
-      }
+      flush_signals(last, w.y, nt, sbuf, rows, sbad, out);
       __syncthreads();
     }
   }
-  if (prow) sbad[g][jj] = bad ? 1 : 0;
-  __syncthreads();
-  if (prow && jj == 0) {
-    int any = 0;
-#pragma unroll
-    for (int j = 0; j < J; ++j) any |= sbad[g][j];
-    status[orow] = any;
-  }
+  if (prow && jj == 0) status[orow] = sbad[g];
 }
 
 // Lanes per problem for S lanes per row: S times the power of two at or
@@ -266,7 +248,7 @@ __global__ __launch_bounds__(kWave) void response_buckets_kernel(
   // loop, so its barriers do not wait on them, and go out coalesced
   __shared__ double2 sbuf[kFlush][kWave / 2];
   __shared__ int64_t rows[kWave / 2];   // output row of each group
-  __shared__ int sbad[kWave / 2][kMaxJ];
+  __shared__ int sbad[kWave / 2];       // a value of the group was not finite
   const int4 w = waves[blockIdx.x];
   // M is the same for every problem of the wavefront; G picks the form:
   // 16 with M + J <= 16 the register-resident one (a problem per 16-lane
