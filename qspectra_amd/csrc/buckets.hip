@@ -136,10 +136,10 @@ __device__ void bucket_wave(const int4 w, const int64_t* __restrict__ offs,
     }
     double2 sum = make_double2((acc[0].x + acc[1].x) + (acc[2].x + acc[3].x),
                                (acc[0].y + acc[1].y) + (acc[2].y + acc[3].y));
-    if (S == 2) {                                        // add the neighbour lane's half
-      sum.x += __shfl_xor(sum.x, 1);
-      sum.y += __shfl_xor(sum.y, 1);
-    }
+    // the neighbour lane's half, within the vector ALU (a wave shuffle's trip
+    // through the LDS crossbar is as long as the product itself)
+    sum.x = seg_sum<S>(sum.x);
+    sum.y = seg_sum<S>(sum.y);
     const int step = k * J + jj;
     if (prow && lead && step < nt) sbuf[step % kFlush][g] = sum;
     if (lead) ys[cur ^ 1][base + i] = sum;
