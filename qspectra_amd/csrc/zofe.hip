@@ -501,6 +501,7 @@ __global__ __launch_bounds__(kColumnThreads) void zofe_column_kernel(
     }
     sites[tid * (1 + S)] = cnt;
   }
+  __syncthreads();      // every wavefront reads the lists in the first stage's (1)
   double2 y[C][N], acc[C][N];
 #pragma unroll
   for (int c = 0; c < C; ++c)
