@@ -189,14 +189,25 @@ def stream_ptr(stream=None):
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    if t is None:
+        return None
+    if t.is_conj() or t.is_neg():
+        raise ValueError('operand is a lazily conjugated or negated view')
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def plain(t):
+    """t contiguous, with its values in memory: kernels read the storage, and
+    contiguous() alone leaves a lazy conjugation (x.conj(), also of a
+    cotangent) or negation (x.conj().imag) pending."""
+    return t.resolve_conj().resolve_neg().contiguous()
 
 
 def to_device(x, dtype=torch.complex128, dev=None):
     """numpy/array-like/tensor -> contiguous device tensor of ``dtype``."""
     dev = device() if dev is None else dev
     if isinstance(x, torch.Tensor):
-        return x.to(device=dev, dtype=dtype).contiguous()
+        return plain(x.to(device=dev, dtype=dtype))
     x = np.ascontiguousarray(x)
     if not x.flags.writeable:              # broadcast views: torch wants writable memory
         x = x.copy()
@@ -353,6 +364,7 @@ def redfield_block_vjp(H1, rw, T, lam, gam, X, Y, flags, unit_convert, gL, strea
     B, n, _ = H1.shape
     assert H1.dtype == torch.float64 and H1.is_contiguous()
     M = block_size(X, n) * block_size(Y, n)
+    gL = gL.resolve_conj()
     assert gL.dtype == torch.complex128 and gL.is_contiguous() and gL.shape == (B, M, M)
     gH1 = torch.empty_like(H1)
     glam = torch.empty((B,), dtype=torch.float64, device=H1.device)
@@ -592,7 +604,7 @@ def propagate_driven(A, col, coef, F, y0, nsub, h, precision=QSX_FP64, diag=None
     if M > MAX_DRIVEN_BLOCK:
         raise ValueError('propagate_driven: block of %d states exceeds %d' % (M, MAX_DRIVEN_BLOCK))
     assert nsub.dtype == torch.int32 and h.dtype == torch.float64
-    A, col, coef, F, y0 = (x.contiguous() for x in (A, col, coef, F, y0))
+    A, col, coef, F, y0 = (plain(x) for x in (A, col, coef, F, y0))
     if col.numel() and (int(col.min()) < 0 or int(col.max()) >= M):
         raise ValueError('propagate_driven: ELL column index outside 0..%d' % (M - 1))
     nF = int(F.shape[1])
@@ -602,7 +614,7 @@ def propagate_driven(A, col, coef, F, y0, nsub, h, precision=QSX_FP64, diag=None
     strideD = 0
     if precision == QSX_MIXED:
         assert diag is not None and diag.dtype == torch.complex128
-        diag = diag.contiguous()
+        diag = plain(diag)
         strideD = 0 if diag.shape[0] == 1 else M
     out = torch.empty((B, R, nsave, M), dtype=torch.complex128, device=y0.device)
     if status is None:
@@ -637,7 +649,7 @@ def propagate_adjoint(A, y0, nsub, total_steps, gout, ckpt=64, stream=None):
         raise ValueError('cotangent shape %s, expected %s' % (tuple(gout.shape),
                                                               (B, R, nsave, M)))
     strideA = 0 if A.shape[0] == 1 else M * M
-    A, y0, gout = A.contiguous(), y0.contiguous(), gout.contiguous()
+    A, y0, gout = plain(A), plain(y0), plain(gout)
     nbytes = lib.qsx_adjoint_workspace_bytes(M, R, B, int(total_steps), int(ckpt))
     if nbytes < 0:
         raise NativeError('invalid adjoint workspace request')
@@ -685,7 +697,7 @@ def _piece_operands(A, y0, sched, v):
         raise ValueError('propagate_pieces: %d states, %d steps' % (M, sched.N))
     if v is not None and (v.dtype != torch.complex128 or tuple(v.shape) != (M,)):
         raise ValueError('propagate_pieces: signal vector of shape %s' % (tuple(v.shape),))
-    return A.contiguous(), y0.contiguous(), None if v is None else v.contiguous()
+    return plain(A), plain(y0), None if v is None else plain(v)
 
 
 def propagate_pieces(A, y0, sched, v=None, stream=None):
@@ -718,7 +730,7 @@ def propagate_pieces_adjoint(A, y0, sched, Q, Y, gout, v=None, stream=None):
     B, R, M = y0.shape
     if tuple(gout.shape) != (B, R, sched.nsave) + (() if v is not None else (M,)):
         raise ValueError('cotangents of shape %s' % (tuple(gout.shape),))
-    gout = gout.contiguous()
+    gout = plain(gout)
     nbytes = lib.qsx_propagate_pieces_adjoint_workspace_bytes(M, R, B, sched.N, sched.len)
     if nbytes < 0:
         raise NativeError('invalid adjoint workspace request')
@@ -758,6 +770,7 @@ def zgemm(A, B, C=None, alpha=1.0, beta=0.0, gamma=0.0, precision=QSX_FP64, stre
     contiguous (for example column slices of a wider matrix)."""
     lib = require_native()
     assert A.dim() == 3 and B.dim() == 3
+    A, B = A.resolve_conj(), B.resolve_conj()
     bA = A.shape[0]
     m, k = (A.shape[2], A.shape[1]) if transa else (A.shape[1], A.shape[2])
     bB = B.shape[0]
@@ -962,7 +975,7 @@ def heom_apply(eom, y, stream=None):
     lib = require_native()
     B = eom.Hop.shape[0]
     assert y.shape == (B, eom.n_ado * eom.M) and y.dtype == torch.complex128
-    y = y.contiguous()
+    y = plain(y)
     out = torch.empty_like(y)
     fn, args = _heom_entry(lib, eom, 'apply')
     check(fn(B, *args, ptr(y), ptr(out), stream_ptr(stream)),
@@ -977,7 +990,7 @@ def heom_propagate(eom, y0, nsub, h, precision=QSX_FP64, want_final=False, strea
     B = eom.Hop.shape[0]
     S = eom.n_ado * eom.M
     assert y0.shape == (B, S) and y0.dtype == torch.complex128
-    y0 = y0.contiguous()
+    y0 = plain(y0)
     nsub = np.ascontiguousarray(nsub, dtype=np.int32)
     h = np.ascontiguousarray(h, dtype=np.float64)
     nsave = int(nsub.size)
@@ -1019,7 +1032,7 @@ def heom_propagate_driven(eom, C, F, y0, nsub, h, precision=QSX_FP64, want_final
     assert F.dtype == torch.complex128 and F.is_contiguous() and F.shape[0] in (1, B)
     P, nF = C.shape[1], F.shape[1]
     assert C.shape[2:] == (M, M) and F.shape[2:] == (3, P)
-    y0 = y0.contiguous()
+    y0 = plain(y0)
     nsub = np.ascontiguousarray(nsub, dtype=np.int32)
     h = np.ascontiguousarray(h, dtype=np.float64)
     nsave = int(nsub.size)
@@ -1064,7 +1077,7 @@ def zofe_apply(eom, y, stream=None):
     layout); returns the derivatives in the same layout."""
     lib = require_native()
     B, R, size = y.shape
-    y = y.contiguous()
+    y = plain(y)
     out = torch.empty_like(y)
     ws = _zofe_ws(lib, B, R, eom, y.device)
     st = lib.qsx_zofe_apply(B, R, eom.N, eom.S, eom.P, *_zofe_common(eom, B), ptr(y), ptr(out),
@@ -1083,15 +1096,15 @@ def zofe_propagate(eom, y0, nsub, h, proj=None, V=None, F=None, stream=None):
     if size != eom.size:
         raise ValueError('ZOFE states have %d elements, the model %d' % (eom.size, size))
     nsave = int(nsub.shape[0])
-    y0 = y0.contiguous()
+    y0 = plain(y0)
     K, strideP = 0, 0
     if proj is not None:
-        proj = proj.contiguous()
+        proj = plain(proj)
         K = int(proj.shape[1])
         strideP = 0 if proj.shape[0] == 1 else K * eom.N * eom.N
     nfield, strideV, strideF, nF = 0, 0, 0, 0
     if V is not None:
-        V, F = V.contiguous(), F.contiguous()
+        V, F = plain(V), plain(F)
         nfield = int(V.shape[1])
         strideV = 0 if V.shape[0] == 1 else nfield * eom.N * eom.N
         nF = int(F.shape[1])
@@ -1118,14 +1131,14 @@ def dense_eigh(H, stream=None):
     qsx_dense_eigh_hermitian, U then complex128."""
     lib = require_native()
     if H.is_complex():
-        H = H.to(torch.complex128).contiguous()
+        H = plain(H.to(torch.complex128))
         B, nb, _ = H.shape
         E = torch.empty((B, nb), dtype=torch.float64, device=H.device)
         U = torch.empty((B, nb, nb), dtype=torch.complex128, device=H.device)
         check(lib.qsx_dense_eigh_hermitian(ptr(H), nb, B, ptr(E), ptr(U), stream_ptr(stream)),
               'qsx_dense_eigh_hermitian')
         return E, U
-    H = H.to(torch.float64).contiguous()
+    H = plain(H.to(torch.float64))
     B, nb, _ = H.shape
     nbytes = lib.qsx_redfield_dense_workspace_bytes(1, nb, nb, B)
     ws = torch.empty((max(nbytes, 8) + 7) // 8, dtype=torch.float64, device=H.device)
@@ -1164,8 +1177,8 @@ def unitary_block_dense(HX, HY, unit_convert, heisenberg=False, stream=None):
     M = nX * nY
     L = torch.empty((B, M, M), dtype=torch.complex128, device=HX.device)
     if HX.is_complex() or HY.is_complex():
-        HX = HX.to(torch.complex128).contiguous()
-        HY = HY.to(torch.complex128).contiguous()
+        HX = plain(HX.to(torch.complex128))
+        HY = plain(HY.to(torch.complex128))
         check(lib.qsx_unitary_block_dense_hermitian(ptr(HX), ptr(HY), nX, nY, B,
                                                     float(unit_convert), int(bool(heisenberg)),
                                                     ptr(L), stream_ptr(stream)),
@@ -1179,7 +1192,7 @@ def unitary_block_dense(HX, HY, unit_convert, heisenberg=False, stream=None):
 
 def _fourier(x, n, N, lo, sign, dt, adjoint, stream):
     lib = require_native()
-    x = x.to(torch.complex128).contiguous()
+    x = plain(x.to(torch.complex128))
     lead = tuple(x.shape[:-1])
     if x.shape[-1] != (N if adjoint else n):
         raise ValueError('fourier transform: last axis has %d entries, expected %d'
@@ -1210,7 +1223,7 @@ def fourier_transform_real(x, N, lo, sign, dt, stream=None):
     batch = int(np.prod(lead)) if lead else 1
     if batch < 2 or not lib.qsx_fourier_real_pairs(int(n), int(N), int(lo)):
         return fourier_transform(x, N, lo, sign, dt, stream).real
-    x = x.to(torch.complex128).contiguous()
+    x = plain(x.to(torch.complex128))
     out = torch.empty(lead + (N,), dtype=torch.float64, device=x.device)
     nbytes = lib.qsx_fourier_workspace_bytes(int(N))
     ws = torch.empty((nbytes + 15) // 16, dtype=torch.complex128, device=x.device)

@@ -49,7 +49,7 @@ class _Propagate(torch.autograd.Function):
         h = torch.ones(len(nsub_host), dtype=torch.float64, device=dev)
         total = int(np.sum(nsub_host))
         states, _, status = _native.propagate_states(
-            _native.QSX_MODE_PROPAGATOR, A.contiguous(), y0.contiguous(), nsub, h,
+            _native.QSX_MODE_PROPAGATOR, _native.plain(A), _native.plain(y0), nsub, h,
             steps=total)
         ctx.save_for_backward(A, y0, nsub)
         ctx.total, ctx.ckpt = total, ckpt
@@ -59,8 +59,7 @@ class _Propagate(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gstates, _gstatus):
         A, y0, nsub = ctx.saved_tensors
-        gA, gy0, status = _native.propagate_adjoint(A, y0, nsub, ctx.total,
-                                                    gstates.contiguous(), ctx.ckpt)
+        gA, gy0, status = _native.propagate_adjoint(A, y0, nsub, ctx.total, gstates, ctx.ckpt)
         if int(status.item()) != 0:
             raise FloatingPointError('adjoint propagation failed (status %d)'
                                      % int(status.item()))
@@ -108,7 +107,7 @@ class _RK4Propagator(torch.autograd.Function):
     @staticmethod
     def forward(ctx, L, h):
         from .lti import rk4_propagator
-        L = L.contiguous()
+        L = _native.plain(L)
         ctx.save_for_backward(L)
         ctx.h = float(h)
         return rk4_propagator(L, ctx.h)
@@ -117,8 +116,8 @@ class _RK4Propagator(torch.autograd.Function):
     def backward(ctx, G):
         (L,) = ctx.saved_tensors
         h = ctx.h
-        G = G.contiguous()
-        X = (L.conj().transpose(-1, -2) * h).contiguous()
+        G = _native.plain(G)
+        X = _native.plain(L.conj().transpose(-1, -2) * h)
         T = G
         Xm = X
         acc = G.clone()
@@ -181,7 +180,7 @@ class _RedfieldBlock(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, H1, lam, rw, T, gamma, X, Y, flags, unit_convert):
-        H1d = H1.detach().contiguous()
+        H1d = _native.plain(H1.detach())
         lam_v = float(lam)
         ctx.args = (rw, T, lam_v, gamma, X, Y, flags, unit_convert)
         ctx.lam_is_tensor = torch.is_tensor(lam)
@@ -193,7 +192,7 @@ class _RedfieldBlock(torch.autograd.Function):
         (H1,) = ctx.saved_tensors
         rw, T, lam, gamma, X, Y, flags, unit_convert = ctx.args
         gH1, glam = _native.redfield_block_vjp(H1, rw, T, lam, gamma, X, Y, flags, unit_convert,
-                                               gL.contiguous())
+                                               _native.plain(gL))
         g_lam = glam.sum() if ctx.lam_is_tensor else None
         return gH1, g_lam, None, None, None, None, None, None, None
 

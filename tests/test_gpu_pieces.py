@@ -109,3 +109,37 @@ def test_pieces_report_non_finite_states(gpu):
     assert int(_native.propagate_pieces(A, y0, sched)[3].item()) == 1
     with pytest.raises(ValueError):
         _native.propagate_pieces(A[:, :2], y0, sched)
+
+
+@pytest.mark.parametrize('M', [5, 20])
+def test_lazily_conjugated_operands_and_cotangents(gpu, M):
+    """gradients.propagate on both routes (16 states at most: pieces) with a
+    loss whose cotangent arrives as a pending conjugation, and operands that
+    are conjugate views, against the recursion in numpy."""
+    A, y0, _ = _problem(M, 2, 2, False, M)
+    nsub = [0] + [1] * 80
+    w = torch.as_tensor(np.random.RandomState(2).normal(size=(2, 2, 81, M)) + 0.5j).to(y0.device)
+    a, y = A.clone().requires_grad_(True), y0.clone().requires_grad_(True)
+    states = G.propagate(a, y, nsub)
+    (w * states.conj()).sum().real.backward()
+    # d Re sum(w conj(s)) with respect to s: w
+    want, gA, gy = _reference(A, y0, nsub, w.cpu().numpy())
+    assert _rel(states, want) <= 1e-11
+    assert _rel(a.grad, gA.sum(axis=1)) <= 1e-11 and _rel(y.grad, gy) <= 1e-11
+    conj = G.propagate(A.conj(), y0.conj(), nsub)
+    assert _rel(conj, want.conj()) <= 1e-11
+
+
+@pytest.mark.parametrize('n', [40, 2500])
+def test_transforms_of_lazily_conjugated_rows(gpu, n):
+    """Forward, real-part and adjoint transforms of x.conj() equal those of
+    the conjugated copy."""
+    x = torch.as_tensor(np.random.RandomState(n).normal(size=(700, n)) + 0.3j).to('cuda')
+    N, lo = 2 * n - 1, n - 1
+    c = x.conj().resolve_conj()
+    for f in (lambda v: _native.fourier_transform(v, N, lo, -1, 0.5),
+              lambda v: _native.fourier_transform_real(v, N, lo, -1, 0.5)):
+        assert torch.equal(f(x.conj()), f(c))
+    g = _native.fourier_transform(x, N, lo, -1, 0.5)
+    assert torch.equal(_native.fourier_transform_adjoint(g.conj(), n, lo, -1, 0.5),
+                       _native.fourier_transform_adjoint(g.conj().resolve_conj(), n, lo, -1, 0.5))

@@ -94,3 +94,25 @@ def test_ctypes_signatures_match_header_prototypes():
             assert a is b, (name, i, a, b)
         want_ret = ctypes.c_int64 if ret == 'int64_t' else ctypes.c_int32
         assert _native.RESTYPES.get(name, ctypes.c_int32) is want_ret, name
+
+
+def test_operands_carry_no_pending_conjugation_or_sign():
+    """Kernels read a tensor's storage: operands are brought to plain memory
+    (contiguous() keeps a lazy conjugation), and a view that still has one
+    pending is refused rather than read without it."""
+    import pytest
+    import torch
+    from qspectra_amd import _native
+    x = torch.tensor([[1 + 2j, 3 - 4j], [5j, -6 + 0j]], dtype=torch.complex128)
+    for view, want in ((x.conj(), [[1 - 2j, 3 + 4j], [-5j, -6]]),
+                       (x.conj().imag, [[-2, 4], [-5, 0]]), (x.t(), [[1 + 2j, 5j], [3 - 4j, -6]])):
+        p = _native.plain(view)
+        assert p.is_contiguous() and not p.is_conj() and not p.is_neg()
+        assert torch.equal(torch.view_as_real(p) if p.is_complex() else p,
+                           torch.view_as_real(torch.tensor(want, dtype=p.dtype))
+                           if p.is_complex() else torch.tensor(want, dtype=p.dtype))
+        assert _native.ptr(p).value == p.data_ptr()
+    for view in (x.conj(), x.conj().imag):
+        with pytest.raises(ValueError):
+            _native.ptr(view)
+    assert not _native.to_device(x.conj(), dev='cpu').is_conj()
