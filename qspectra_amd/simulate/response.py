@@ -15,7 +15,6 @@ Keyword options in addition to the reference's: ``dt`` (RK4 step),
 ``plan`` ('fused', the default, see fused.py; or 'pathways', one pathway at a
 time as the reference does).
 """
-import copy
 
 import numpy as np
 import torch
@@ -25,7 +24,7 @@ from .decorators import (optional_ensemble_average, optional_2nd_order_isotropic
                          optional_4th_order_isotropic_average)
 from .utils import propagate, propagate_heom, propagate_zofe, fourier_transform
 from ..dynamics.heom import DeviceHEOM
-from ..utils import ZeroArray
+from ..utils import ZeroArray, copy_with_new_cache
 
 _PROPAGATE_KW = ('dt', 'precision', 'rtol', 'schedule')
 
@@ -41,8 +40,7 @@ def _members(model):
 
 
 def _member_model(model, ham):
-    m = copy.copy(model)
-    m.__dict__.pop('_imemoize__cache', None)
+    m = copy_with_new_cache(model)
     m.__dict__.pop('_batch', None)
     m.hamiltonian = ham
     return m

@@ -54,10 +54,17 @@ def memoized_property(func):
     return property(imemoize(func))
 
 
+# where objects keep what they have derived from their attributes
+_DERIVED = ('_imemoize__cache', '_eoms', '_builder_inputs')
+
+
 def copy_with_new_cache(obj):
-    """Shallow copy without the imemoize cache (qspectra/utils.py:98-108)."""
+    """Shallow copy without what the object has derived from its attributes:
+    the imemoize cache (qspectra/utils.py:98-108) and a model's equations of
+    motion and builder inputs, which hold its Hamiltonians."""
     new = copy.copy(obj)
-    new.__dict__.pop('_imemoize__cache', None)
+    for name in _DERIVED:
+        new.__dict__.pop(name, None)
     return new
 
 

@@ -285,3 +285,22 @@ def test_heom_fields_match_oracle_and_reference(gpu):
     t, y = qa.simulate_pump(mp, pp, 'x', time_extra=10., liouville_subspace='gg', dt=dt)
     to, yo = P.simulate_pump(mo, po, 'x', time_extra=10., liouville_subspace='gg', dt=dt)
     assert rel_err(np.asarray(y), yo) < 1e-10
+
+
+def test_ensemble_of_a_model_that_has_been_used(gpu):
+    """The ensemble average does not depend on whether the model has
+    propagated its own Hamiltonian before."""
+    rho0 = np.zeros((2, 2))
+    rho0[1, 1] = 1
+    t = np.arange(0, 20.0, 1.0)
+    out = []
+    for used in (False, True):
+        ham = qa.ElectronicHamiltonian(np.array([[12000., 50.], [50., 12100.]]),
+                                       bath=qa.DebyeBath(53.5, 35., 106.), dipoles=np.eye(2, 3),
+                                       disorder=100., random_seed=0)
+        m = qa.HEOMModel(ham, rw_freq=12000., hilbert_subspace='ge', unit_convert=qa.CM_FS,
+                         level_cutoff=3, K=1)
+        if used:
+            qa.simulate_dynamics(m, rho0, times=t, dt=0.5)
+        out.append(qa.simulate_dynamics(m, rho0, times=t, ensemble_size=3, dt=0.5)[1])
+    assert np.array_equal(*out)

@@ -298,3 +298,27 @@ def test_arbitrary_bath_host():
     assert not hasattr(b, 'corr_func_complex')
     assert b.spectral_density_limit_at_zero == 2 * lam / gam
     assert not qa.bath.is_debye_form(b)
+
+
+@pytest.mark.parametrize('kind', ['redfield', 'heom', 'zofe'])
+def test_copies_with_other_hamiltonians_keep_nothing_derived(kind):
+    """A model that has been used hands neither its equations of motion nor
+    its builder inputs (they hold its Hamiltonian) to the batched and sampled
+    copies made from it."""
+    bath = qa.DebyeBath(53.5, 35., 106.)
+    if kind == 'zofe':
+        one = np.ones((1, 2))
+        bath = qa.PseudomodeBath(1, 100. * one + 0j, 50. * one + 0j, 0.1 * one + 0j)
+    ham = qa.ElectronicHamiltonian(np.array([[12000., 50.], [50., 12100.]]), bath=bath,
+                                   dipoles=np.eye(2, 3), disorder=100., random_seed=0)
+    kw = dict(rw_freq=12000., hilbert_subspace='ge', unit_convert=qa.CM_FS)
+    model = {'redfield': lambda: qa.RedfieldModel(ham, **kw),
+             'heom': lambda: qa.HEOMModel(ham, level_cutoff=2, K=1, **kw),
+             'zofe': lambda: qa.ZOFEModel(ham, **kw)}[kind]()
+    for name in ('_imemoize__cache', '_eoms', '_builder_inputs'):
+        model.__dict__[name] = {'used': 1}
+    members = [h.in_rotating_frame(12000.) for h in ham.sample_ensemble(2)]
+    for new in [model.with_hamiltonians(members)] + list(model.sample_ensemble(2)):
+        assert not any('used' in (new.__dict__.get(name) or {})
+                       for name in ('_imemoize__cache', '_eoms', '_builder_inputs'))
+    assert model.__dict__['_eoms'] == {'used': 1}
