@@ -189,18 +189,16 @@ def stream_ptr(stream=None):
 
 
 def ptr(t):
-    if t is None:
-        return None
-    if t.is_conj() or t.is_neg():
-        raise ValueError('operand is a lazily conjugated or negated view')
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
 def plain(t):
     """t contiguous, with its values in memory: kernels read the storage, and
     contiguous() alone leaves a lazy conjugation (x.conj(), also of a
     cotangent) or negation (x.conj().imag) pending."""
-    return t.resolve_conj().resolve_neg().contiguous()
+    if t.is_conj() or t.is_neg():
+        t = t.resolve_conj().resolve_neg()
+    return t.contiguous()
 
 
 def to_device(x, dtype=torch.complex128, dev=None):
@@ -770,7 +768,7 @@ def zgemm(A, B, C=None, alpha=1.0, beta=0.0, gamma=0.0, precision=QSX_FP64, stre
     contiguous (for example column slices of a wider matrix)."""
     lib = require_native()
     assert A.dim() == 3 and B.dim() == 3
-    A, B = A.resolve_conj(), B.resolve_conj()
+    A, B = (X.resolve_conj() if X.is_conj() else X for X in (A, B))
     bA = A.shape[0]
     m, k = (A.shape[2], A.shape[1]) if transa else (A.shape[1], A.shape[2])
     bB = B.shape[0]
