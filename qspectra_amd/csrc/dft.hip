@@ -24,10 +24,18 @@
 // one complex multiply-add per sample) and R = 1, 2 or 4 batch rows (the
 // twiddles are the rows'): 4 + 4 / R FP64 operations per sample for two
 // outputs, where one output of one row took 8.  The rows are staged through
-// LDS in tiles (every thread reads the same sample: broadcast).  Four chains
-// of twiddles, each advanced by four samples' step, hide their latency.
-// Measured (129 rows of 1000 samples onto 1999 points): 68 us, with one
-// output of one row per thread and the samples staged in LDS 136 us.
+// LDS in tiles (every thread reads the same sample: broadcast), 8 KB per
+// work-group whatever R, and a launch has threads for the pairs that have an
+// output only, in work-groups of whole wavefronts: short grids (up to 127
+// points: one wavefront) and the adjoints of short signals far from t = 0 keep
+// twenty work-groups on a CU.  Four chains of twiddles, each advanced by four
+// samples' step, hide their latency.
+// Measured (host call): 129 rows of 1000 samples onto 1999 points 67 us, with
+// one output of one row per thread 122 us; 20000 rows of 61 samples onto 121
+// points 26 us, the adjoint 41 us, with N / 2 + 1 pairs in work-groups of 256
+// and 32 KB of samples 64 and 112 us, with one output per thread 76 and 94 us;
+// adjoint of 3000 rows from 4000 points to 100 samples at their end 446, 4402
+// and 677 us.
 //
 // Long transforms (both lengths >= kChirpMin) take Bluestein's chirp-z form
 // instead, O(N log N) per row.  Both directions are one sum
@@ -61,8 +69,8 @@ namespace qsx {
 namespace {
 
 constexpr int kDftThreads = 256;
-constexpr int kDftTile = 512;
-constexpr int kAnchor = 16;   // samples between exact twiddles (divides kDftTile)
+constexpr int kDftTile = 512;  // samples in LDS, of all R rows together
+constexpr int kAnchor = 16;   // samples between exact twiddles (divides kDftTile / R)
 
 __global__ __launch_bounds__(kDftThreads) void dft_twiddle_kernel(int N, double2* __restrict__ T) {
   const int m = blockIdx.x * kDftThreads + threadIdx.x;
@@ -78,19 +86,25 @@ __device__ inline int64_t mod_n(int64_t a, int64_t N) {
 }
 
 // out[b, u] = scale * sum_v in[b, v] * T[(a_u * d_v) mod N] (conj if adj),
-// a_u = a0 + da * u, d_v = d0 + dd * v.  Thread q <= N/2 forms the outputs
-// with a_u = q and a_u = -q (mod N), where they exist, of R rows.
+// a_u = a0 + da * u, d_v = d0 + dd * v.  A thread forms the outputs with
+// a_u = q and a_u = -q (mod N), where they exist, of R rows, for its one of the
+// nq values q = q0, q0 + 1, .. <= N/2 that have any.  Wavefronts beyond them
+// only stage samples.
 template <int R>
 __global__ __launch_bounds__(kDftThreads) void dft_kernel(
     const double2* __restrict__ in, int64_t batch, int n_in, int n_out, int N, int64_t a0,
-    int da, int64_t d0, int dd, int adj, double scale, const double2* __restrict__ T,
-    double2* __restrict__ out) {
-  __shared__ double2 xs[R][kDftTile];
-  const int64_t q = (int64_t)blockIdx.x * kDftThreads + threadIdx.x;
-  const int64_t a = min(q, (int64_t)(N / 2));
+    int da, int64_t d0, int dd, int q0, int nq, int adj, double scale,
+    const double2* __restrict__ T, double2* __restrict__ out) {
+  constexpr int kTile = kDftTile / R;
+  __shared__ double2 xs[R][kTile];
+  const int nt = blockDim.x;
+  const int64_t q = (int64_t)blockIdx.x * nt + threadIdx.x;
+  const bool mine = q < nq, busy = __any(mine);
+  const int64_t a = q0 + min(q, (int64_t)(nq - 1));
   const int64_t u0 = mod_n(da * (a - a0), N), u1 = mod_n(da * (-a - a0), N);
-  const bool w0 = q <= N / 2 && u0 < n_out, w1 = q <= N / 2 && u1 < n_out && u1 != u0;
-  const int step = (int)mod_n(a * dd, N), anchor_step = (int)mod_n((int64_t)step * kAnchor, N);
+  const bool w0 = mine && u0 < n_out, w1 = mine && u1 < n_out && u1 != u0;
+  const int step = (int)mod_n(a * dd, N);
+  const int anchor_step = (int)mod_n((int64_t)step * kAnchor, N);
   const int m0 = (int)mod_n(a * mod_n(d0, N), N);
   const double sg = adj ? -1.0 : 1.0;
   const double2 w = make_double2(T[step].x, sg * T[step].y), w2 = cmul(w, w), w4 = cmul(w2, w2);
@@ -99,17 +113,19 @@ __global__ __launch_bounds__(kDftThreads) void dft_kernel(
 #pragma unroll
     for (int r = 0; r < R; ++r) rr[r] = ii[r] = ri[r] = ir[r] = 0.0;
     int m = m0;
-    for (int v0 = 0; v0 < n_in; v0 += kDftTile) {
-      const int len = min(kDftTile, n_in - v0);
+    for (int v0 = 0; v0 < n_in; v0 += kTile) {
+      const int len = min(kTile, n_in - v0);
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const double2* row = in + min(b0 + r, batch - 1) * n_in + v0;
-        for (int k = threadIdx.x; k < len; k += kDftThreads) xs[r][k] = row[k];
+        for (int k = threadIdx.x; k < len; k += nt) xs[r][k] = row[k];
       }
       __syncthreads();
-      // exact twiddle from the table every kAnchor samples, in between
-      // multiplied by step twiddles (error <= kAnchor / 4 + 4 rounding steps)
+      // exact twiddle from the table every kAnchor samples, in between multiplied
+      // by step twiddles: with one rounding error for a table entry and one for
+      // a product, w, w2 and w4 carry 1, 3 and 7 of them, t[3] starts with 7, and
+      // each of its three products with w4 adds 8: at most 31 (first order)
       auto samples = [&](int k0, int count, auto full) {
         constexpr bool FULL = decltype(full)::value;
         double2 t[4];
@@ -135,6 +151,7 @@ __global__ __launch_bounds__(kDftThreads) void dft_kernel(
         m += anchor_step;
         if (m >= N) m -= N;
       };
+      if (!busy) continue;
       int k0 = 0;
       for (; k0 + kAnchor <= len; k0 += kAnchor) samples(k0, kAnchor, std::true_type());
       if (k0 < len) samples(k0, len - k0, std::false_type());
@@ -743,14 +760,23 @@ extern "C" int32_t qsx_fourier_transform(const void* x, int64_t batch, int32_t n
   }
   hipLaunchKernelGGL(dft_twiddle_kernel, dim3((N + kDftThreads - 1) / kDftThreads), dim3(kDftThreads),
                      0, s, N, T);
-  // more rows per thread while that leaves two work-groups for every CU
-  const int64_t gx = (N / 2 + kDftThreads) / kDftThreads;
-  const int R = gx * ((batch + 3) / 4) >= 512 ? 4 : (gx * ((batch + 1) / 2) >= 256 ? 2 : 1);
+  // the pairs q = |a| of the outputs' a = a0 .. a0 + da (n_out - 1), which lie in
+  // [-N/2, N/2]: all of 0 .. N/2 forward, the samples' own in the adjoint
+  const int64_t a1 = a0 + (int64_t)da * (n_out - 1);
+  const int64_t amin = std::min(a0, a1), amax = std::max(a0, a1);
+  const int q0 = (int)(amin > 0 ? amin : (amax < 0 ? -amax : 0));
+  const int nq = (int)std::max(-amin, amax) - q0 + 1;
+  // equal work-groups of whole wavefronts; more rows per thread while that
+  // leaves two wavefronts (four rows) or one (two rows) for every SIMD
+  const int64_t gx = (nq + kDftThreads - 1) / kDftThreads;
+  const int waves = (int)(((nq + gx - 1) / gx + 63) / 64);
+  const int R = gx * waves * ((batch + 3) / 4) >= 2048 ? 4
+              : (gx * waves * ((batch + 1) / 2) >= 1024 ? 2 : 1);
   const auto kern = R == 4 ? dft_kernel<4> : (R == 2 ? dft_kernel<2> : dft_kernel<1>);
   const unsigned gy = (unsigned)std::min<int64_t>((batch + R - 1) / R, 65535);
-  hipLaunchKernelGGL(kern, dim3((unsigned)gx, gy), dim3(kDftThreads), 0, s,
-                     static_cast<const double2*>(x), batch, n_in, n_out, N, a0, da, d0, dd,
-                     (int)(adjoint != 0), dt, T, static_cast<double2*>(out));
+  hipLaunchKernelGGL(kern, dim3((unsigned)gx, gy), dim3(64 * waves), 0, s,
+                     static_cast<const double2*>(x), batch, n_in, n_out, N, a0, da, d0, dd, q0,
+                     nq, (int)(adjoint != 0), dt, T, static_cast<double2*>(out));
   QSX_CHECK_HIP(hipGetLastError());
   return QSX_OK;
 }

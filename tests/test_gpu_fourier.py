@@ -100,11 +100,15 @@ def test_long_rows_forward_and_adjoint(gpu, n, t0, dt, rows):
 
 @pytest.mark.parametrize('rows,n,lo,N', [(1, 1, 0, 1), (2, 2, 1, 4), (3, 17, 0, 33), (5, 16, 15, 31),
                                          (5, 600, 599, 1199), (700, 300, 0, 600),
-                                         (2100, 70, 69, 139), (1, 513, 100, 1024)])
+                                         (2100, 70, 69, 139), (1, 513, 100, 1024),
+                                         (9, 40, 300, 1000), (3, 40, 700, 1000),
+                                         (2100, 100, 1400, 1500), (700, 257, 0, 514),
+                                         (2, 64, 63, 127), (4200, 65, 64, 129)])
 def test_direct_sum_row_groups(gpu, rows, n, lo, N):
     """The direct sum over one, two and four rows per thread, odd and even
     grids, sample counts that are no multiple of the twiddle block or tile,
-    placed anywhere on the grid: against the sum in numpy, forward (both
+    placed anywhere on the grid (also all before or all after its zero), pair
+    counts at the edges of a wavefront and a work-group: against the sum in numpy, forward (both
     signs) and adjoint.  n products of unit twiddles accurate to a few ulp:
     1e-12 of the row's scale."""
     rs = np.random.RandomState(n)
