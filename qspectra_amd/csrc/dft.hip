@@ -104,15 +104,16 @@ __global__ __launch_bounds__(kDftThreads) void dft_kernel(
   const int64_t u0 = mod_n(da * (a - a0), N), u1 = mod_n(da * (-a - a0), N);
   const bool w0 = mine && u0 < n_out, w1 = mine && u1 < n_out && u1 != u0;
   const int step = (int)mod_n(a * dd, N);
-  const int anchor_step = (int)mod_n((int64_t)step * kAnchor, N);
-  const int m0 = (int)mod_n(a * mod_n(d0, N), N);
+  // unsigned: two residues add up to less than 2^32
+  const unsigned anchor_step = (unsigned)mod_n((int64_t)step * kAnchor, N);
+  const unsigned m0 = (unsigned)mod_n(a * mod_n(d0, N), N);
   const double sg = adj ? -1.0 : 1.0;
   const double2 w = make_double2(T[step].x, sg * T[step].y), w2 = cmul(w, w), w4 = cmul(w2, w2);
   for (int64_t b0 = (int64_t)blockIdx.y * R; b0 < batch; b0 += (int64_t)gridDim.y * R) {
     double rr[R], ii[R], ri[R], ir[R];       // sums of x.x t.x, x.y t.y, x.x t.y, x.y t.x
 #pragma unroll
     for (int r = 0; r < R; ++r) rr[r] = ii[r] = ri[r] = ir[r] = 0.0;
-    int m = m0;
+    unsigned m = m0;
     for (int v0 = 0; v0 < n_in; v0 += kTile) {
       const int len = min(kTile, n_in - v0);
       __syncthreads();
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(kDftThreads) void dft_kernel(
           }
         }
         m += anchor_step;
-        if (m >= N) m -= N;
+        if (m >= (unsigned)N) m -= N;
       };
       if (!busy) continue;
       int k0 = 0;

@@ -150,3 +150,22 @@ def test_paired_real_parts(gpu, rows, n, sign):
             assert np.isnan(got[b]).all()
         else:
             assert np.abs(got[b] - want[b]).max() <= 1e-13 * np.abs(want[b]).max()
+
+
+def test_direct_sum_on_a_grid_beyond_2_30_points(gpu):
+    """Twiddle indices of a grid whose residues' sums pass 2^31: 48 samples
+    (three exact twiddles each) onto 2^30 + 5 points, a few of the outputs
+    against the sum in numpy with exponents reduced in Python integers."""
+    N, n, lo = (1 << 30) + 5, 48, 12345
+    if torch.cuda.get_device_properties(0).total_memory < 48 << 30:
+        pytest.skip('needs 35 GB of device memory')
+    rs = np.random.RandomState(0)
+    x = rs.normal(size=n) + 1j * rs.normal(size=n)
+    out = _native.fourier_transform(torch.as_tensor(x).to('cuda'), N, lo, -1, 0.5)
+    c = N // 2
+    at = np.concatenate([[0, 1, 2, N - 1, c - 1, c, c + 1], rs.randint(0, N, 200)])
+    got = out[torch.as_tensor(at).to('cuda')].cpu().numpy()
+    del out
+    want = [0.5 * sum(x[j] * np.exp(-2j * np.pi * (((int(r) - c) * (lo + j - c)) % N) / N)
+                      for j in range(n)) for r in at]
+    assert np.abs(got - want).max() <= 1e-12 * np.abs(x).sum()
