@@ -346,14 +346,28 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // MIXED; 74 and 66 us when every edge was gathered, all products were complex
 // and stages wrote separate stage vectors (55 and 62 us with the existing
 // edges alone).  In FP64 a stage now moves 210 MB (FETCH_SIZE, WRITE_SIZE) at
-// 4.3 TB/s, where a device copy reaches 5.1.  Six wavefronts per SIMD (a few
-// spilled registers) beat five by 3% and 8%; holding an element's operator
-// entries in registers, nested brackets y + h/m A (..) in place of the series
-// terms, and non-temporal loads and stores were slower.
+// 4.3 TB/s, where a device copy reaches 5.1.  Nested brackets y + h/m A (..)
+// in place of the series terms and non-temporal loads and stores were slower.
 // TIN: the type of the stage's input (MIXED: double for the series' first
 // stage, whose input is y).
+//
+// Registers.  Where M divides the work-group (4 and 8 states) a thread's elements
+// share their row and column, and the compiler holds the operator's row and
+// column in registers: at 8 states 4 wavefronts per SIMD for one Matsubara term
+// and 3 for two leave room for that (132 and 140 registers), and it is the
+// fastest; below, the element index is kept opaque so that the entries stay in
+// LDS and 6 (5) wavefronts fit in 80 (96) registers with at most 4 spilled.
+// Measured against one bound of 6 (4 for two terms) at every size: 8 sites, 969
+// ADOs, 48 samples, 20 steps 7.6 -> 3.6 ms FP64 and 6.0 -> 3.6 MIXED for a real
+// Hamiltonian, 3.5 for a complex one (24 samples took 7.7), 75 to 100 registers
+// spilled before; 7 sites, 2024 ADOs, two terms 7.0 -> 6.0 and 5.8 -> 5.5; 7
+// sites, one term unchanged.
+constexpr int comm_waves(int nX, int kb) {
+  return nX == 8 ? (kb == 2 ? 4 : 3) : (kb == 2 ? 6 : 5);
+}
+
 template <typename T, typename TIN, int NX, int NY, int NR, int KB>
-__global__ __launch_bounds__(kThreads, KB == 2 ? 6 : 4) void heom_comm_kernel(
+__global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel(
     HeomArgs a, const void* __restrict__ zin_, cplx_t<T>* __restrict__ zout,
     HeomStageBufs<T> bf, double h, int st) {
   using T2 = cplx_t<TIN>;
@@ -422,7 +436,9 @@ __global__ __launch_bounds__(kThreads, KB == 2 ? 6 : 4) void heom_comm_kernel(
   auto elements = [&](auto form) {
     constexpr bool GENERAL = decltype(form)::value;
     for (int e = tid; e < nloc * M; e += kThreads) {
-      const int la = e / M, p = e - la * M, ado = ado0 + la;
+      int eo = e;
+      if (NX < 8) asm volatile("" : "+v"(eo));     // see the registers above
+      const int la = eo / M, p = eo - la * M, ado = ado0 + la;
       const int r = p % NX, c = p / NX;
       const double2* z = zt + la * M;
       // per occupied-site slot: the neighbour gathers of the edges that exist,
