@@ -54,6 +54,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kXcds = 8;
+constexpr int kCUs = 256;
 #ifndef QSX_HEOM_ELEMS_PER_THREAD
 #define QSX_HEOM_ELEMS_PER_THREAD 3
 #endif
@@ -602,6 +603,43 @@ inline int heom_samples_per_pass(int B, int64_t bytes_per_sample) {
   return std::min(B, c);
 }
 
+inline void set_tile(HeomArgs& a, int elems) {
+  a.ado_per_tile = std::max(1, elems * kThreads / a.M);
+  a.tiles = (a.n_ado + a.ado_per_tile - 1) / a.ado_per_tile;
+}
+
+// Elements per thread (1 .. kElemsPerThread) for launches of B samples: the
+// fewest rounds of work-groups on the chip, each priced at its elements per
+// thread and half an element for the operators and tables it sets up.  Returns
+// the kernel's dynamic LDS bytes.
+// Measured (20 steps, us FP64 / MIXED at three, two and one): 7 sites, 3060 ADOs,
+// 4 samples (0.5, 0.8, 1.6 rounds) 1210 / 1290, 1165 / 1120, 1240 / 1150; 8
+// samples (1.1, 1.6, 3.2) 1870 / 1735, 1705 / 1660 (two); 2024 ADOs, two terms, 4
+// samples (0.4, 0.6, 1.3) 1250 / 1440, 985 / 1120, 1010 / 1035, 8 samples (0.8,
+// 1.3, 2.5) 1310 / 1310, 1485 / 1425, 1375 / 1370; 5 sites, 1001 ADOs, 48
+// samples (1.1, 1.6, 3.2) 1840 / 1635, 1565 / 1460 (two).  One element per thread
+// only below 512 work-groups, as before, took three for all of these.
+inline size_t choose_tile(HeomArgs& a, int B, const void* kern, size_t elem_bytes) {
+  int64_t best = INT64_MAX;
+  int pick = kElemsPerThread;
+  for (int elems = kElemsPerThread; elems >= 1; --elems) {
+    set_tile(a, elems);
+    const size_t lds = heom_lds_bytes(heom_opsz(a), a.ado_per_tile, a.M, a.nbins, elem_bytes, a.N);
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kThreads, lds) != hipSuccess)
+      (void)hipGetLastError();
+    if (per_cu < 1) break;              // the launch's own checks report it
+    const int64_t slots = (int64_t)kCUs * per_cu;
+    const int64_t cost = ((int64_t)B * a.tiles + slots - 1) / slots * (2 * elems + 1);
+    if (cost < best) {
+      best = cost;
+      pick = elems;
+    }
+  }
+  set_tile(a, pick);
+  return heom_lds_bytes(heom_opsz(a), a.ado_per_tile, a.M, a.nbins, elem_bytes, a.N);
+}
+
 // workspace bytes per hierarchy element: FP64 y and three terms or stage
 // vectors; MIXED y and in complex64 three terms, or with stage vectors its
 // copy, z2..z4 and k1..k3
@@ -610,7 +648,7 @@ inline int64_t heom_bytes_per_element(bool fp64, bool series) {
 }
 
 template <typename T>
-int run_heom(const HeomArgs& a0, const double2* y0, const int32_t* nsub, const double* h,
+int run_heom(HeomArgs a0, const double2* y0, const int32_t* nsub, const double* h,
              int nsave, double2* out, double2* yfin, void* workspace, int* status,
              hipStream_t stream, const HeomFields& fl = HeomFields()) {
   using T2 = cplx_t<T>;
@@ -633,11 +671,11 @@ int run_heom(const HeomArgs& a0, const double2* y0, const int32_t* nsub, const d
   // then z[1..3]
   const void* zins[4] = {kFp64 || series ? (const void*)bf.y : bf.z[0], bf.z[1], bf.z[2], bf.z[3]};
   const int opsz = heom_opsz(a0);
-  const size_t shmem = heom_lds_bytes(opsz, a0.ado_per_tile, a0.M, a0.nbins,
-                                       is_comm_shape(a0) ? sizeof(double2) : sizeof(T2), a0.N);
-  QSX_CHECK_ARG(shmem <= 160 * 1024, "qsx_heom_propagate: %zu bytes of LDS", shmem);
   const StageKernel<T> kern = pick_stage_kernel<T>(a0);
   const StageKernel<T> first = series ? pick_stage_kernel<T, double>(a0) : kern;
+  const size_t shmem = choose_tile(a0, Bc, (const void*)kern,
+                                   is_comm_shape(a0) ? sizeof(double2) : sizeof(T2));
+  QSX_CHECK_ARG(shmem <= 160 * 1024, "qsx_heom_propagate: %zu bytes of LDS", shmem);
   if (shmem > 64 * 1024)
     for (const StageKernel<T> k : {kern, first})
       QSX_CHECK_HIP(hipFuncSetAttribute((const void*)k,
@@ -721,13 +759,7 @@ static int fill_args(qsx::HeomArgs& a, int B, int n_ado, int M, int n, const voi
   a.nbins = nbins;
   a.K1 = K1;
   a.nrel = nrel;
-  // fewer elements per thread while the launch would not give every CU two
-  // work-groups (one 3060-ADO hierarchy: 204 work-groups at 3, 612 at 1)
-  for (int elems = kElemsPerThread; elems >= 1; --elems) {
-    a.ado_per_tile = std::max(1, elems * kThreads / M);
-    a.tiles = (n_ado + a.ado_per_tile - 1) / a.ado_per_tile;
-    if ((int64_t)B * a.tiles >= 512) break;
-  }
+  set_tile(a, kElemsPerThread);
   a.xcd_map = B >= kXcds;
   a.Hop = (const double2*)Hop;
   a.shift = shift;
@@ -743,13 +775,12 @@ static int fill_args(qsx::HeomArgs& a, int B, int n_ado, int M, int n, const voi
   return QSX_OK;
 }
 
-static int heom_apply_impl(const qsx::HeomArgs& a, const void* y, void* out, void* stream) {
+static int heom_apply_impl(qsx::HeomArgs a, const void* y, void* out, void* stream) {
   using namespace qsx;
   QSX_CHECK_ARG(y && out, "qsx_heom_apply: null pointer");
-  const int opsz = heom_opsz(a);
-  const size_t shmem = heom_lds_bytes(opsz, a.ado_per_tile, a.M, a.nbins, sizeof(double2), a.N);
-  QSX_CHECK_ARG(shmem <= 160 * 1024, "qsx_heom_apply: %zu bytes of LDS", shmem);
   const StageKernel<double> kern = pick_stage_kernel<double>(a);
+  const size_t shmem = choose_tile(a, a.B, (const void*)kern, sizeof(double2));
+  QSX_CHECK_ARG(shmem <= 160 * 1024, "qsx_heom_apply: %zu bytes of LDS", shmem);
   if (shmem > 64 * 1024)
     QSX_CHECK_HIP(hipFuncSetAttribute((const void*)kern,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));

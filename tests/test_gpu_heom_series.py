@@ -56,3 +56,36 @@ def test_commutator_form_matches_rk4(gpu, sites, K, levels, members, imag):
             assert np.abs(whole.cpu().numpy() - want).max() <= tol * np.abs(want).max()
             ado0 = propagate_heom(eom, yd, t, dt=dt, precision=precision).cpu().numpy()
             assert np.abs(ado0 - want[:, :, :eom.M]).max() <= tol * np.abs(want).max()
+
+
+@pytest.mark.parametrize('sites,K,levels,members', [
+    (2, 1, 4, 3), (5, 1, 4, 60), (7, 2, 3, 30), (8, 1, 3, 70), (8, 2, 3, 9)])
+def test_batches_match_their_members(gpu, sites, K, levels, members):
+    """Real and complex Hamiltonians in one batch, at batch sizes whose launches
+    give a thread one, two and three elements, against batches of one: the
+    same sums in the same order, so the same bits."""
+    rs = np.random.RandomState(sites + members)
+    bath = DebyeBath(CM_K * 300, 35., 106.)
+    hams = []
+    for imag in (0, 1, 0):
+        J = np.triu(rs.normal(0, 60, (sites, sites)) + imag * 1j * rs.normal(0, 60, (sites, sites)),
+                    1)
+        hams.append(ElectronicHamiltonian(J + J.conj().T + np.diag(rs.uniform(12200, 12700, sites)),
+                                          bath=bath, dipoles=np.ones((sites, 3)))
+                    .in_rotating_frame(12450.))
+    model = HEOMModel(hams[0], rw_freq=12450., hilbert_subspace='ge', unit_convert=CM_FS,
+                      level_cutoff=levels, K=K)
+    pick = rs.randint(0, 3, members)
+    pick[:3] = 0, 1, 2
+    batch = model.with_hamiltonians([hams[i] for i in pick]).equation_of_motion('ee')
+    y0 = rs.normal(size=(3, batch.size)) + 1j * rs.normal(size=(3, batch.size))
+    y0 = torch.as_tensor(y0).to(batch.Hop.device)
+    t = np.array([0.0, 2.0])
+    for precision in ('fp64', 'mixed'):
+        got = propagate_heom(batch, y0[pick], t, dt=0.5, precision=precision, full_states=True)
+        for i in range(3):
+            one = model.with_hamiltonians([hams[i]]).equation_of_motion('ee')
+            want = propagate_heom(one, y0[i:i + 1], t, dt=0.5, precision=precision,
+                                  full_states=True)
+            for b in np.flatnonzero(pick == i):
+                assert torch.equal(got[b], want[0]), (precision, i, b)
