@@ -436,6 +436,9 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
   const T2* zb = zin + (int64_t)b * a.n_ado * M;
   auto elements = [&](auto form) {
     constexpr bool GENERAL = decltype(form)::value;
+    // gathers in flight: of all slots where the registers allow it (the small
+    // hierarchies of 2 and 3 states wait for their latency), else of one
+    constexpr int SLOTS = NX <= 3 ? NR : 1;
     for (int e = tid; e < nloc * M; e += kThreads) {
       int eo = e;
       if (NX < 8) asm volatile("" : "+v"(eo));     // see the registers above
@@ -443,26 +446,34 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
       const int r = p % NX, c = p / NX;
       const double2* z = zt + la * M;
       // per occupied-site slot: the neighbour gathers of the edges that exist,
-      // in flight during a half of the commutator
+      // in flight during the commutator or a half of it
       const double2* tc = tcf + la * nb2;
       const double2 zp = z[p];
       double2 k = cmul(make_double2(a.shift[ado] + a.dvec[p].x, a.dvec[p].y), zp);
-#pragma unroll
-      for (int t = 0; t < NR; ++t) {
+      int src[SLOTS][2 * KB];
+      T2 v[SLOTS][2 * KB];
+      auto gather = [&](int t) {
         const int2* ts = reinterpret_cast<const int2*>(tsrc + la * nb2 + pbin[p][t]);
-        int src[2 * KB];
-        T2 v[2 * KB];
+        const int u = SLOTS == 1 ? 0 : t;
 #pragma unroll
         for (int kk = 0; kk < KB; ++kk) {
           const int2 sk = ts[kk];
-          src[2 * kk] = sk.x;
-          src[2 * kk + 1] = sk.y;
+          src[u][2 * kk] = sk.x;
+          src[u][2 * kk + 1] = sk.y;
         }
 #pragma unroll
         for (int o = 0; o < 2 * KB; ++o) {
-          v[o] = T2{0, 0};
-          if (src[o] >= 0) v[o] = zb[src[o] * M + p];
+          v[u][o] = T2{0, 0};
+          if (src[u][o] >= 0) v[u][o] = zb[src[u][o] * M + p];
         }
+      };
+      if (SLOTS > 1)
+#pragma unroll
+        for (int t = 0; t < NR; ++t) gather(t);
+#pragma unroll
+      for (int t = 0; t < NR; ++t) {
+        const int u = SLOTS == 1 ? 0 : t;
+        if (SLOTS == 1) gather(t);
         // (H_X rho - rho H_Y)_{rc}, p = r + NX c, column-major rho
         if (t == 0) {
 #pragma unroll
@@ -482,8 +493,8 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
         }
 #pragma unroll
         for (int o = 0; o < 2 * KB; ++o) {
-          if (src[o] >= 0) {
-            const double2 cf = tc[pbin[p][t] + o], x = to_d2(v[o]);
+          if (src[u][o] >= 0) {
+            const double2 cf = tc[pbin[p][t] + o], x = to_d2(v[u][o]);
             if (o % 2 == 0) {
               const double w = pwp[p][t];
               if (GENERAL) cfma<double>(k, make_double2(cf.x * w, cf.y * w), x);
