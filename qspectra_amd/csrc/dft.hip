@@ -530,7 +530,8 @@ __global__ __launch_bounds__(kFftThreads) void chirp_rows_kernel(
 // forward and two inverse FFTs per chunk, and the output is written as
 // doubles.  Row b is scaled by a power of two to row a's magnitude (each
 // row's rounding error stays relative to its own); rows that cannot share
-// (non-finite, zero, or beyond the exponent range) are transformed one by one:
+// (non-finite, zero, row a beyond 2^+-500 or the rows that far apart) are
+// transformed one by one:
 // row a in the first launch, which marks row b for the second (ALONE).
 // Bound by the FFT passes (LDS and FP64 issue, one work-group per CU).
 // Measured (5120 rows of 4096 samples onto 8191 points): 530 + 6 us; row by
@@ -584,8 +585,10 @@ __global__ __launch_bounds__(kFftThreads) void chirp_pairs_kernel(
       mb = fmax(mb, smax[1][q]);
     }
     shift = __builtin_amdgcn_readfirstlane(ma > 0.0 && mb > 0.0 ? ilogb(ma) - ilogb(mb) : 0);
+    // row b takes row a's magnitude: away from both ends of the exponent range,
+    // so that it neither overflows nor loses bits where it would not alone
     share = __builtin_amdgcn_readfirstlane(rb < batch && all_finite && ma > 0.0 && mb > 0.0 &&
-                                           abs(shift) < 500);
+                                           abs(ilogb(ma)) < 500 && abs(shift) < 500);
   }
   // the power of two of each row (0: not in it)
   const double fa = ALONE ? 0.0 : 0.5, fb = ALONE ? 0.5 : (share ? ldexp(0.5, shift) : 0.0);

@@ -169,3 +169,23 @@ def test_direct_sum_on_a_grid_beyond_2_30_points(gpu):
     want = [0.5 * sum(x[j] * np.exp(-2j * np.pi * (((int(r) - c) * (lo + j - c)) % N) / N)
                       for j in range(n)) for r in at]
     assert np.abs(got - want).max() <= 1e-12 * np.abs(x).sum()
+
+
+@pytest.mark.parametrize('a,b', [(1e306, 1e200), (1e-300, 1e-200), (1e-310, 1.0), (1e160, 1e10),
+                                 (1e140, 1e290), (1e-140, 1e-290)])
+def test_paired_rows_at_the_ends_of_the_exponent_range(gpu, a, b):
+    """A row beside one that overflows or is almost denormal: its real part is
+    that of the row alone (1e-13 of its own scale, as above)."""
+    rs = np.random.RandomState(3)
+    n = 2100
+    N, lo = 2 * n - 1, n - 1
+    x = rs.normal(size=(2, n)) + 1j * rs.normal(size=(2, n))
+    xd = torch.as_tensor(x * [[a], [b]]).to('cuda')
+    got = _native.fourier_transform_real(xd, N, lo, -1, 0.5).cpu().numpy()
+    with np.errstate(over='ignore', invalid='ignore'):
+        want = _native.fourier_transform(torch.as_tensor(x).to('cuda'), N, lo, -1,
+                                         0.5).real.cpu().numpy() * [[a], [b]]
+    for g, w in zip(got, want):
+        if 1e-290 < np.abs(w).max() < 1e305:
+            assert np.isfinite(g).all()
+            assert np.abs(g - w).max() <= 1e-13 * np.abs(w).max()
