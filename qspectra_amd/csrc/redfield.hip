@@ -467,20 +467,21 @@ __global__ __launch_bounds__(NT) void block_rec_kernel(const double* __restrict_
 }
 
 // The records of one or two blocks of B problems.
-void launch_recs(const double* H1, int n, int B, const double* rw, double T, double lam,
-                 double gam, int real_corr, const RecJob* jobs, int njobs, size_t rstride,
-                 int eig_only, hipStream_t s) {
+int launch_recs(const double* H1, int n, int B, const double* rw, double T, double lam,
+                double gam, int real_corr, const RecJob* jobs, int njobs, size_t rstride,
+                int eig_only, hipStream_t s) {
   const RecJob j1 = jobs[njobs - 1];
   const int nb = std::max(jobs[0].nb, j1.nb), m = nb + (nb & 1);
   const bool wide = nb > kWideBlock;
   // sized by the blocks at hand: small ones fill a CU's threads, not its LDS
   const size_t lds = 2 * (size_t)m * m * sizeof(double);
   if (lds > 60 * 1024)
-    (void)hipFuncSetAttribute((const void*)block_rec_kernel<kWideThreads>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    QSX_CHECK_HIP(hipFuncSetAttribute((const void*)block_rec_kernel<kWideThreads>,
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const auto kern = wide ? block_rec_kernel<kWideThreads> : block_rec_kernel<kThreads>;
   hipLaunchKernelGGL(kern, dim3(B, njobs), dim3(wide ? kWideThreads : kThreads), lds, s, H1, n,
                      rw, T, lam, gam, real_corr, jobs[0], j1, rstride, eig_only);
+  return QSX_OK;
 }
 
 // sandwich: out[i + nX j] = sum_{a,b} UX[i][a] Z[a + nX b] UY[j][b]  (LDS)
@@ -1527,7 +1528,8 @@ extern "C" int32_t qsx_block_eigh(const double* H1, int32_t n, int32_t B, int32_
   double* ws = static_cast<double*>(workspace);
   hipStream_t s = as_stream(stream);
   const RecJob job = {nullptr, nullptr, nullptr, ws, X, nb};
-  launch_recs(H1, n, B, rw, 1.0, 0.0, 1.0, 0, &job, 1, rs, 1, s);
+  st = launch_recs(H1, n, B, rw, 1.0, 0.0, 1.0, 0, &job, 1, rs, 1, s);
+  if (st) return st;
   QSX_CHECK_HIP(hipGetLastError());
   QSX_CHECK_HIP(hipMemcpy2DAsync(E, nb * sizeof(double), ws, rs * sizeof(double),
                                  nb * sizeof(double), B, hipMemcpyDeviceToDevice, s));
@@ -1579,7 +1581,9 @@ static int redfield_block_impl(const double* H1, int n, int B, const double* rw,
   double2* W = reinterpret_cast<double2*>(wsX + 2 * rs * B);
   const RecJob jobs[2] = {{nullptr, nullptr, static_cast<const double2*>(ctabX), wsX, X, nX},
                           {nullptr, nullptr, static_cast<const double2*>(ctabY), wsY, Y, nY}};
-  launch_recs(H1, n, B, rw, T, lam, gam, (flags & kRealCorr) != 0, jobs, X == Y ? 1 : 2, rs, 0, s);
+  const int st = launch_recs(H1, n, B, rw, T, lam, gam, (flags & kRealCorr) != 0, jobs,
+                             X == Y ? 1 : 2, rs, 0, s);
+  if (st) return st;
   // non-secular blocks whose transformed factors fit the LDS: one pass
   const size_t kron = kron_lds_bytes(n, nX, nY);
   if (!(flags & kSecular) && n <= kKronMaxSites && kron <= 160 * 1024) {
@@ -1642,7 +1646,8 @@ extern "C" int32_t qsx_dense_eigh(const double* H, int32_t nb, int32_t B, double
   double* ws = static_cast<double*>(workspace);
   hipStream_t s = as_stream(stream);
   const RecJob job = {H, nullptr, nullptr, ws, 0, nb};
-  launch_recs(nullptr, 1, B, nullptr, 1.0, 0.0, 1.0, 0, &job, 1, rs, 1, s);
+  const int st = launch_recs(nullptr, 1, B, nullptr, 1.0, 0.0, 1.0, 0, &job, 1, rs, 1, s);
+  if (st) return st;
   QSX_CHECK_HIP(hipGetLastError());
   QSX_CHECK_HIP(hipMemcpy2DAsync(E, nb * sizeof(double), ws, rs * sizeof(double),
                                  nb * sizeof(double), B, hipMemcpyDeviceToDevice, s));
@@ -1672,8 +1677,9 @@ extern "C" int32_t qsx_redfield_block_dense(const double* HX, const double* HY, 
   double2* W = reinterpret_cast<double2*>(wsX + 2 * rs * B);
   hipStream_t s = as_stream(stream);
   const RecJob jobs[2] = {{HX, occX, nullptr, wsX, 0, nX}, {HY, occY, nullptr, wsY, 0, nY}};
-  launch_recs(nullptr, n, B, nullptr, T, lam, gam, (flags & kRealCorr) != 0, jobs, same ? 1 : 2, rs,
-              0, s);
+  const int st = launch_recs(nullptr, n, B, nullptr, T, lam, gam, (flags & kRealCorr) != 0, jobs,
+                             same ? 1 : 2, rs, 0, s);
+  if (st) return st;
   const size_t shmem = 3 * (size_t)M * sizeof(double2) + (size_t)(nX * nX + nY * nY) * sizeof(double);
   QSX_CHECK_ARG(shmem <= 64 * 1024, "qsx_redfield_block_dense: block too large (M=%d)", M);
   hipLaunchKernelGGL(liouv_cols_kernel, dim3(M, B), dim3(kThreads), shmem, s, n, nX, nY,
@@ -1772,7 +1778,9 @@ extern "C" int32_t qsx_redfield_block_vjp(const double* H1, int32_t n, int32_t B
   const size_t cstride = vjp_slab_doubles(std::max(nX, nY));
   const RecJob jobs[2] = {{nullptr, nullptr, nullptr, wsX, X, nX},
                           {nullptr, nullptr, nullptr, wsY, Y, nY}};
-  launch_recs(H1, n, B, rw, T, lam, gam, (flags & kRealCorr) != 0, jobs, same ? 1 : 2, rs, 0, s);
+  st = launch_recs(H1, n, B, rw, T, lam, gam, (flags & kRealCorr) != 0, jobs,
+                   same ? 1 : 2, rs, 0, s);
+  if (st) return st;
   const double2* G = static_cast<const double2*>(gL);
   if (!(flags & kEigenBasis)) {
     hipLaunchKernelGGL(vjp_cols_kernel, dim3(M, B), dim3(kThreads), shmem, s, n, nX, nY, wsX,

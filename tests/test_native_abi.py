@@ -111,3 +111,14 @@ def test_operands_carry_no_pending_conjugation_or_sign():
                            if p.is_complex() else torch.tensor(want, dtype=p.dtype))
         assert _native.ptr(p).value == p.data_ptr()
     assert not _native.to_device(x.conj(), dev='cpu').is_conj()
+
+
+def test_no_hip_status_is_dropped():
+    """hipFuncSetAttribute reports an LDS size the device does not have; every
+    call in the sources goes through the status check."""
+    from qspectra_amd.csrc import build as B
+    for fn in sorted(os.listdir(B.HERE)):
+        if fn.endswith('.hip'):
+            text = open(os.path.join(B.HERE, fn)).read()
+            for m in re.finditer(r'hipFuncSetAttribute\(', text):
+                assert text[:m.start()].endswith('QSX_CHECK_HIP('), (fn, m.start())
