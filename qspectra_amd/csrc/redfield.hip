@@ -387,7 +387,9 @@ __device__ void block_bath(int n, const RecJob& job, double T, double lam, doubl
     const int c = d + r;
     const double x = rec.E[d] - rec.E[c];
     const bool sum = !real_corr && x != 0.0;
-    double2 M = sum ? matsubara_partial(x, T, gam, 1 + sub, S) : make_double2(0.0, 0.0);
+    double2 M = make_double2(0.0, 0.0);
+    if (sum)          // constant strides where one lane has the whole sum
+      M = S == 1 ? matsubara_partial(x, T, gam, 1, 1) : matsubara_partial(x, T, gam, 1 + sub, S);
     for (int o = 1; o < S; o *= 2) {
       M.x += __shfl_xor(M.x, o);
       M.y += __shfl_xor(M.y, o);
@@ -1030,9 +1032,13 @@ __global__ __launch_bounds__(NT) void absorption_ops_kernel(
 
 // C(x)/lam and dC/dx of the Debye bath (the x = 0 branch is a constant), by
 // S neighbouring lanes (a power of two, sub = 0 .. S - 1, the same x): each
-// takes every S-th term of the two sums
+// takes every S-th term of the two sums.  ONE: S = 1, its strides constant
+// (blocks of 12 states and more; with the loops' strides in a register the
+// reverse mode of a block of 21 took 777 us for 733)
+template <bool ONE>
 __device__ void debye_corr_grad(double x, double T, double lam, double gam, int real_corr,
-                                int sub, int S, double2& c1, double2& dc) {
+                                int sub_, int S_, double2& c1, double2& dc) {
+  const int sub = ONE ? 0 : sub_, S = ONE ? 1 : S_;
   if (real_corr) {
     if (x == 0.0) {
       c1 = make_double2(T * 2.0 / gam, 0.0);
@@ -1310,7 +1316,10 @@ __global__ __launch_bounds__(kThreads) void vjp_chain_kernel(
   for (int e0 = 0; e0 < nb2; e0 += kThreads / S) {
     const int e = min(e0 + tid / S, nb2 - 1), d = e / nb, c = e % nb;
     double2 c1, dc;
-    debye_corr_grad(r.E[d] - r.E[c], T, lam, gam, real_corr, tid & (S - 1), S, c1, dc);
+    if (S == 1)
+      debye_corr_grad<true>(r.E[d] - r.E[c], T, lam, gam, real_corr, 0, 1, c1, dc);
+    else
+      debye_corr_grad<false>(r.E[d] - r.E[c], T, lam, gam, real_corr, tid & (S - 1), S, c1, dc);
     if ((tid & (S - 1)) != 0 || e0 + tid / S >= nb2) continue;
     C1[e] = c1;
     dC[e] = dc;
