@@ -1730,10 +1730,13 @@ extern "C" int32_t qsx_absorption_operators(const int64_t* table, int32_t B, int
   // rounds but leave fewer compute units to the other size classes and the
   // propagation running beside them.  One wavefront up to eight sites, where a
   // Jacobi round has at most 48 items: its barriers cost nothing and four times
-  // as many problems share the chip.  Few problems keep 256 threads for the
-  // summed Matsubara form of baths outside the closed form's range.
-  const auto kern = max_n <= 8 && B >= 64 ? absorption_ops_kernel<64> : absorption_ops_kernel<256>;
-  const int threads = max_n <= 8 && B >= 64 ? 64 : 256;
+  // as many problems share the chip.  That pays from two problems per CU on;
+  // below, 256 threads are as fast (8 sites, 448 problems, whole ensemble pass
+  // 110 us for 106) and share the Matsubara sums of baths outside the closed
+  // form's range, where one wavefront took 147 us for 125.
+  const bool narrow = max_n <= 8 && B >= 512;
+  const auto kern = narrow ? absorption_ops_kernel<64> : absorption_ops_kernel<256>;
+  const int threads = narrow ? 64 : 256;
   if (lds > 64 * 1024)
     QSX_CHECK_HIP(hipFuncSetAttribute((const void*)kern,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
