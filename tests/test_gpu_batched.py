@@ -293,3 +293,39 @@ def test_absorption_operators_match_block_builder(gpu, secular, real, bath):
             assert rel_err(P1[o:o + n * n].reshape(n, n), ref1[s][k]) < 1e-12, (n, k)
             assert rel_err(PJ[o:o + n * n].reshape(n, n), refJ[s][k]) < 1e-12, (n, k)
             row += 1
+
+
+@pytest.mark.parametrize('bath', [BATH, NARROW_WARM, BROAD_COLD])
+@pytest.mark.parametrize('problems', [511, 512, 700])
+def test_absorption_operators_of_many_small_problems(gpu, bath, problems):
+    """1..8 sites on both sides of the count from which a wavefront has a
+    problem of its own, the Matsubara sum in closed form or summed: the
+    operators of the same problems in a launch of eight (1e-12, as above)."""
+    import torch
+    rs = np.random.RandomState(problems)
+    H1, table, oh, op = [], [], 0, 0
+    for n in range(1, 9):
+        J = np.triu(rs.normal(0, 60, (n, n)), 1)
+        H1.append((J + J.T + np.diag(rs.uniform(12200, 12700, n))).ravel())
+        table.append((n, oh, op))
+        oh += n * n
+        op += n * n
+    pick = rs.randint(0, 8, problems)
+    many, o = [], 0
+    for k in pick:
+        many.append((table[k][0], table[k][1], o))
+        o += table[k][0] ** 2
+    out = []
+    for tb, size in ((table, op), (many, o)):
+        P = [torch.zeros(size, dtype=torch.complex128, device='cuda') for _ in range(2)]
+        _native.absorption_operators_into(
+            torch.as_tensor(np.asarray(tb, dtype=np.int64)).cuda(), 8,
+            torch.as_tensor(np.concatenate(H1)).cuda(),
+            torch.full((len(tb),), 12450.0, dtype=torch.float64, device='cuda'),
+            torch.as_tensor(np.tile(bath, (len(tb), 1)).astype(float)).cuda(), 8, qa.CM_FS, 1.0, 4,
+            *P)
+        out.append([p.cpu().numpy() for p in P])
+    for few, lots in zip(*out):
+        want = np.concatenate([few[table[k][2]:table[k][2] + table[k][0] ** 2] for k in pick])
+        assert np.abs(want).max() > 0
+        assert rel_err(lots, want) < 1e-12
