@@ -1213,13 +1213,24 @@ def fourier_transform(x, N, lo, sign, dt, stream=None):
     return _fourier(x, x.shape[-1], N, lo, sign, dt, False, stream)
 
 
-def fourier_transform_real(x, N, lo, sign, dt, stream=None):
-    """The real part of fourier_transform: float64 [..., N] (two rows per
-    transform where qsx_fourier_real_pairs takes the sizes)."""
+def real_pairs_pay(rows):
+    """Whether that many rows go through the paired transform.  A work-group
+    (one per CU, 256 at a time) takes 5/3 as long for a pair as for a row (50
+    and 31 us per round at 4096 samples, 31 and 18 at 2048), so pairs pay where
+    they save rounds: 256 rows of 4096 samples 74 us paired and 59 single, 300
+    rows 73 and 85, 600 rows 120 and 115, 1024 rows 126 and 148."""
+    return 5 * -(-rows // 512) < 3 * -(-rows // 256)
+
+
+def fourier_transform_real(x, N, lo, sign, dt, stream=None, pairs=None):
+    """The real part of fourier_transform: float64 [..., N], two rows per
+    transform where qsx_fourier_real_pairs takes the sizes and real_pairs_pay
+    the row count (pairs: the latter's choice when given)."""
     lib = require_native()
     n, lead = x.shape[-1], tuple(x.shape[:-1])
     batch = int(np.prod(lead)) if lead else 1
-    if batch < 2 or not lib.qsx_fourier_real_pairs(int(n), int(N), int(lo)):
+    if batch < 2 or not (real_pairs_pay(batch) if pairs is None else pairs) or \
+            not lib.qsx_fourier_real_pairs(int(n), int(N), int(lo)):
         return fourier_transform(x, N, lo, sign, dt, stream).real
     x = plain(x.to(torch.complex128))
     out = torch.empty(lead + (N,), dtype=torch.float64, device=x.device)

@@ -143,7 +143,7 @@ def test_paired_real_parts(gpu, rows, n, sign):
         x[2, 7] = np.nan
     xd = torch.as_tensor(x).to('cuda')
     want = _native.fourier_transform(xd, N, lo, sign, 0.5).real.cpu().numpy()
-    got = _native.fourier_transform_real(xd, N, lo, sign, 0.5).cpu().numpy()
+    got = _native.fourier_transform_real(xd, N, lo, sign, 0.5, pairs=True).cpu().numpy()
     assert got.dtype == np.float64 and got.shape == (rows, N)
     for b in range(rows):
         if np.isnan(x[b]).any():
@@ -181,7 +181,7 @@ def test_paired_rows_at_the_ends_of_the_exponent_range(gpu, a, b):
     N, lo = 2 * n - 1, n - 1
     x = rs.normal(size=(2, n)) + 1j * rs.normal(size=(2, n))
     xd = torch.as_tensor(x * [[a], [b]]).to('cuda')
-    got = _native.fourier_transform_real(xd, N, lo, -1, 0.5).cpu().numpy()
+    got = _native.fourier_transform_real(xd, N, lo, -1, 0.5, pairs=True).cpu().numpy()
     with np.errstate(over='ignore', invalid='ignore'):
         want = _native.fourier_transform(torch.as_tensor(x).to('cuda'), N, lo, -1,
                                          0.5).real.cpu().numpy() * [[a], [b]]

@@ -122,3 +122,12 @@ def test_no_hip_status_is_dropped():
             text = open(os.path.join(B.HERE, fn)).read()
             for m in re.finditer(r'hipFuncSetAttribute\(', text):
                 assert text[:m.start()].endswith('QSX_CHECK_HIP('), (fn, m.start())
+
+
+def test_row_counts_of_the_paired_transform():
+    """Up to 256 rows every row has a CU of its own: pairs would run longer.
+    From there they pay where they save a round of work-groups."""
+    from qspectra_amd import _native
+    for rows, pay in ((1, False), (2, False), (256, False), (257, True), (512, True),
+                      (513, False), (768, False), (769, True), (1024, True), (5120, True)):
+        assert _native.real_pairs_pay(rows) is pay, rows
