@@ -8,6 +8,7 @@ There is no CPU fallback: every compute entry point raises
 ``NativeUnavailable`` when the library or a HIP device is missing.
 """
 import ctypes
+import math
 import os
 import threading
 
@@ -668,19 +669,26 @@ def propagate_adjoint(A, y0, nsub, total_steps, gout, ckpt=64, stream=None):
 MAX_PIECE_STATES = 16
 
 
+def piece_length(steps):
+    """Steps per piece: the power of two next to sqrt(steps), 8..64."""
+    return 1 << min(6, max(3, math.ceil(math.log2(max(steps, 1)) / 2)))
+
+
 class PieceSchedule(object):
     """Device tables of qsx_propagate_pieces for step counts nsub (host) of
     the save intervals: the step after which each save is taken, cut into
-    pieces of ``len`` steps (the power of two next to sqrt(N), 8..64)."""
+    pieces of ``len`` steps (piece_length)."""
 
     def __init__(self, nsub, dev):
         pos = np.cumsum(np.maximum(np.asarray(nsub, dtype=np.int64).reshape(-1), 0))
         self.N, self.nsave = int(pos[-1]), len(pos)
-        self.len = int(2 ** np.clip(np.ceil(np.log2(np.sqrt(max(self.N, 1)))), 3, 6))
+        self.len = piece_length(self.N)
         self.np = -(-self.N // self.len)
-        first = np.searchsorted(pos, self.len * np.arange(self.np), side='right')
-        table = np.concatenate([pos, first, [self.nsave]]).astype(np.int32)
-        table = torch.as_tensor(table).to(dev)
+        table = np.empty(self.nsave + self.np + 1, dtype=np.int32)
+        table[:self.nsave] = pos
+        table[self.nsave:-1] = np.searchsorted(pos, np.arange(0, self.N, self.len), side='right')
+        table[-1] = self.nsave
+        table = torch.from_numpy(table).to(dev)
         self.pos, self.first = table[:self.nsave], table[self.nsave:]
 
 

@@ -135,23 +135,36 @@ def rk4_propagator(L, h):
     return _RK4Propagator.apply(L, h)
 
 
-# steps from which the recursion is cut into pieces: below, a chain of N steps
-# is no longer than the pieces' extra launches
-PIECE_STEPS = 64
+# steps from which the recursion is cut into pieces, where its gradient is
+# needed and where not.  Measured, ratio of the step-by-step recursion's time (2
+# to 16 states, 1 to 8192 right-hand sides): forward and reverse 0.92-1.4 at 64
+# steps, 1.0-2.2 at 96, 1.1-2.4 at 128; forward alone 0.97-1.3 at 96, 1.02-1.5
+# at 128 with up to 8 states.  Pieces double the forward products, which at
+# more states fill the chip earlier: with 12 and 16 states and 2048 right-hand
+# sides 0.85-1.1 up to 256 steps, 1.1-1.8 at 512.
+PIECE_STEPS = 96
+PIECE_STEPS_FORWARD = 128
+PIECE_STEPS_WIDE = 512          # forward alone, more than 8 states,
+PIECE_WIDE_RHS = 1024           # this many right-hand sides
 # memory of the reverse pass's partial gradients (one M x M block per piece):
 # beyond it, right-hand sides alone fill the chip
 PIECE_BYTES = 1 << 29
 
 
-def _pieces(M, rhs, nsub, dev, signal=False):
+def _pieces(M, rhs, nsub, dev, signal=False, grad=True):
     """The PieceSchedule serving rhs right-hand sides of M states over the
     save intervals nsub, or None where the step-by-step recursion does."""
     if M > _native.MAX_PIECE_STATES - bool(signal):
         return None
-    if not PIECE_STEPS <= int(np.sum(np.maximum(nsub, 0))) < 1 << 24:
+    steps = int(np.maximum(nsub, 0).sum())
+    least = (PIECE_STEPS if grad else PIECE_STEPS_WIDE if M > 8 and rhs >= PIECE_WIDE_RHS
+             else PIECE_STEPS_FORWARD)
+    if not least <= steps < 1 << 24:
         return None
-    sched = _native.PieceSchedule(nsub, dev)
-    return sched if 16 * rhs * sched.np * M * (M + 2) <= PIECE_BYTES else None
+    pieces = -(-steps // _native.piece_length(steps))
+    if 16 * rhs * pieces * M * (M + 2) > PIECE_BYTES:
+        return None
+    return _native.PieceSchedule(nsub, dev)
 
 
 def propagate(A, y0, nsub, ckpt=64):
@@ -160,7 +173,8 @@ def propagate(A, y0, nsub, ckpt=64):
     The reverse pass recomputes the forward states from checkpoints every
     ckpt steps (blocks up to M = 160; at most 16 states: from the starts of
     the pieces the steps are cut into, see _native.PieceSchedule)."""
-    sched = _pieces(y0.shape[-1], y0.shape[0] * y0.shape[1], nsub, y0.device)
+    grad = torch.is_grad_enabled() and (A.requires_grad or y0.requires_grad)
+    sched = _pieces(y0.shape[-1], y0.shape[0] * y0.shape[1], nsub, y0.device, grad=grad)
     if sched is not None:
         states, status = _PropagatePieces.apply(A, y0, sched, None)
     else:

@@ -117,8 +117,8 @@ def test_lazily_conjugated_operands_and_cotangents(gpu, M):
     loss whose cotangent arrives as a pending conjugation, and operands that
     are conjugate views, against the recursion in numpy."""
     A, y0, _ = _problem(M, 2, 2, False, M)
-    nsub = [0] + [1] * 80
-    w = torch.as_tensor(np.random.RandomState(2).normal(size=(2, 2, 81, M)) + 0.5j).to(y0.device)
+    nsub = [0] + [1] * 100
+    w = torch.as_tensor(np.random.RandomState(2).normal(size=(2, 2, 101, M)) + 0.5j).to(y0.device)
     a, y = A.clone().requires_grad_(True), y0.clone().requires_grad_(True)
     states = G.propagate(a, y, nsub)
     (w * states.conj()).sum().real.backward()

@@ -78,3 +78,43 @@ def test_site_hamiltonian_and_disorder_shifts():
     shifts = G.disorder_shifts(4, 100, 5, random_seed=7)
     for n, member in enumerate(ham.sample_ensemble(5)):
         assert np.allclose(member.H_1exc, H + np.diag(shifts[n]), rtol=0, atol=1e-12)
+
+
+def test_piece_tables():
+    """Save positions and per-piece save counts of qsx_propagate_pieces against
+    a walk over the steps."""
+    from qspectra_amd import _native
+    for nsub in ([8], [9], [0] + [1] * 64, [0, 0, 3, 0, 70, 1, 1, 0, 0, 40], [130, 0, 0],
+                 [0] + [1] * 4095, [5, 60, 0, 2] + [7] * 30):
+        s = _native.PieceSchedule(np.array(nsub), 'cpu')
+        pos, at = [], 0
+        for n in nsub:
+            at += n
+            pos.append(at)
+        assert s.N == at and s.len in (8, 16, 32, 64) and s.np == -(-at // s.len)
+        assert s.len ** 2 >= min(at, 64 ** 2) and (s.len == 8 or (s.len // 2) ** 2 < at)
+        assert s.pos.tolist() == pos
+        first = [sum(p <= j * s.len for p in pos) for j in range(s.np)] + [len(pos)]
+        assert s.first.tolist() == first
+
+
+def test_route_of_the_propagation(monkeypatch):
+    """Pieces from the measured step counts on, and no tables built for a call
+    that keeps the step-by-step recursion."""
+    from qspectra_amd import _native, gradients as G
+
+    class Tables(object):
+        def __init__(self, nsub, dev):
+            built.append(len(nsub))
+    monkeypatch.setattr(_native, 'PieceSchedule', Tables)
+    for M, rhs, steps, grad, signal, want in (
+            (7, 512, 96, True, False, True), (7, 512, 95, True, False, False),
+            (7, 512, 127, False, False, False), (7, 512, 128, False, False, True),
+            (16, 1023, 128, False, False, True), (16, 1024, 511, False, False, False),
+            (16, 1024, 512, False, False, True), (16, 1024, 96, True, False, True),
+            (17, 1, 500, True, False, False), (16, 1, 500, True, True, False),
+            (15, 1, 500, True, True, True), (16, 8192, 512, True, False, False),
+            (2, 1 << 20, 96, True, False, False)):
+        built = []
+        got = G._pieces(M, rhs, [steps], 'cpu', signal=signal, grad=grad)
+        assert (got is not None) == bool(built) == want, (M, rhs, steps, grad, signal)
