@@ -143,3 +143,22 @@ def test_transforms_of_lazily_conjugated_rows(gpu, n):
     g = _native.fourier_transform(x, N, lo, -1, 0.5)
     assert torch.equal(_native.fourier_transform_adjoint(g.conj(), n, lo, -1, 0.5),
                        _native.fourier_transform_adjoint(g.conj().resolve_conj(), n, lo, -1, 0.5))
+
+
+def test_powers_that_overflow_where_no_state_does(gpu):
+    """A mode that grows by 1e6 a step and is not in the states: its 64th power
+    overflows, the states and gradients of the recursion are finite; with it
+    in the states both routes report it."""
+    A = torch.diag(torch.tensor([1e6, 0.9], dtype=torch.complex128)).to('cuda')[None]
+    y0 = torch.tensor([[[0, 1 + 1j]]], dtype=torch.complex128, device='cuda')
+    nsub = [0] + [1] * 300
+    a, y = A.clone().requires_grad_(True), y0.clone().requires_grad_(True)
+    states = G.propagate(a, y, nsub)
+    (states[..., 1].abs() ** 2).sum().backward()
+    g = np.zeros((1, 1, 301, 2), dtype=complex)
+    g[0, 0, :, 1] = 2 * (1 + 1j) * 0.9 ** np.arange(301)
+    want, gA, gy = _reference(A, y0, nsub, g)
+    assert _rel(states, want) <= 1e-11
+    assert _rel(a.grad, gA.sum(axis=1)) <= 1e-11 and _rel(y.grad, gy) <= 1e-11
+    with pytest.raises(FloatingPointError):
+        G.propagate(A, torch.ones_like(y0), nsub)
