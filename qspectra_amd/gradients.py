@@ -156,7 +156,7 @@ def _pieces(M, rhs, nsub, dev, signal=False, grad=True):
     save intervals nsub, or None where the step-by-step recursion does."""
     if M > _native.MAX_PIECE_STATES - bool(signal):
         return None
-    steps = int(np.maximum(nsub, 0).sum())
+    steps = int(np.asarray(nsub).sum())
     least = (PIECE_STEPS if grad else PIECE_STEPS_WIDE if M > 8 and rhs >= PIECE_WIDE_RHS
              else PIECE_STEPS_FORWARD)
     if not least <= steps < 1 << 24:
