@@ -540,7 +540,8 @@ int32_t qsx_propagate_driven(int32_t precision, const void* A, int64_t strideA,
  *           couplings, zofe.py:214-215; strideL)
  *   Gamma, w  [B|1][P][S] Omega^2 huang and i Omega + gamma (strideG)
  *   flags   bit 0 ham_hermit, bit 1 rho_hermit (zofe.py:170-186); bit 2: every
- *           L_s is diagonal (off-diagonal entries are then not read)
+ *           L_s is diagonal (its off-diagonal entries must be zero: some
+ *           kernels read them, some do not)
  *   nfield, V [B|1][nfield][N][N], F [B|1][nF][3][nfield]: field terms
  *   y0      [B][R][N^2 (1 + P S)] states in the reference's layout (vec of
  *           rho, then vec of O with shape (P, S, N, N), both column-major)

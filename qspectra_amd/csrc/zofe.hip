@@ -390,8 +390,8 @@ __global__ __launch_bounds__(NT) void zofe_kernel(ZofeArgs a, const double2* __r
 //       is read once for all C columns, the entries of be's column k are
 //       spread over the 16 lanes of each row and broadcast from there (DPP),
 //       so a column costs N^2 / C + 4 N LDS reads of 16 B where the
-//       element-wise kernel takes 4 N per element; the threads of the last
-//       wavefront derive one element of rho each, its sums over sites again
+//       element-wise kernel takes 4 N per element; eight lanes derive each
+//       element of rho, one term of its sums per lane, those over sites again
 //       only over the sites that couple;
 //   (3) the RK4 update written back into LDS.
 // Measured (7 sites, 16 modes, one right-hand side): 8.2 us per stage, with
@@ -804,25 +804,35 @@ static int32_t zofe_launch(int apply,
   a.strideP = strideP;
   hipStream_t st = as_stream(stream);
   dim3 grid(R, B);
-  // the column form wherever its threads and LDS suffice: 2.0 times as fast
-  // as the element-wise kernel at 7 sites and 16 modes.  One column per thread
-  // while that takes at most one wavefront per SIMD, two beyond (each row of X
-  // then read once for both; one column in 128 registers measured 13.2 us per
-  // stage against 8.2 us)
+  // the column form wherever its threads and LDS suffice: 2.1 times as fast
+  // as the element-wise kernel at 7 sites and 16 modes (20 steps 615 us for
+  // 1300), 1.05 to 3.4 times over 1..8 states and 1..16 modes, one right-hand side
+  // or 300.  One column per thread while that takes at most one wavefront per
+  // SIMD, two beyond (each row of X then read once for both; one column in 128
+  // registers measured 13.2 us per stage against 8.2 us).  At 6 and 7 states it
+  // holds one work-group per CU (122 and 147 us per 256 right-hand sides and 8
+  // steps) where the element-wise kernel with few modes holds up to four: from
+  // two to four rounds on that one is taken (8 steps, 1024 right-hand sides, column /
+  // element-wise: 6 states, P S = 5, 10, 12, 20: 481 / 290, 487 / 351, 491 / 401,
+  // 499 / 467; 7 states, P S = 6: 593 / 451, P S = 12 the column form 1.3 times
+  // as fast).
   const int cols = (P * S * N <= 256) ? 1 : 2, need = P * S * ((N + cols - 1) / cols);
   const size_t cshmem = zofe_column_lds_bytes(N, S, P);
+  const int64_t groups = (int64_t)R * B;
+  const bool crowded = (N == 6 && groups > (P * S <= 5 ? 256 : P * S <= 12 ? 512 : 768) &&
+                        P * S <= 20) || (N == 7 && P * S <= 6 && groups > 768);
   if (!apply && (flags & kZofeDiagonal) && N <= 8 && need <= kColumnThreads &&
-      cshmem <= 160 * 1024) {
+      cshmem <= 160 * 1024 && !crowded) {
     const int nt = (std::max(need, 8 * N * N) + 63) / 64 * 64;    // <= kColumnThreads
 #define QSX_ZOFE_COLUMN(N_, C_)                                                                \
   if (N == N_ && cols == C_) {                                                                 \
-    auto kern = nfield ? zofe_column_kernel<N_, C_, true> : zofe_column_kernel<N_, C_, false>;                                                    \
+    auto kern = nfield ? zofe_column_kernel<N_, C_, true> : zofe_column_kernel<N_, C_, false>; \
     if (cshmem > 64 * 1024)                                                                    \
       QSX_CHECK_HIP(hipFuncSetAttribute((const void*)kern,                                     \
                                         hipFuncAttributeMaxDynamicSharedMemorySize,            \
                                         (int)cshmem));                                         \
     hipLaunchKernelGGL(kern, grid, dim3(nt), cshmem, st, a, (const double2*)y0, nsub, h,       \
-                       nsave, (double2*)out, status);                                    \
+                       nsave, (double2*)out, status);                                          \
     QSX_CHECK_HIP(hipGetLastError());                                                          \
     return QSX_OK;                                                                             \
   }

@@ -94,3 +94,24 @@ def test_first_stage_does_not_depend_on_what_the_lds_held(gpu):
             assert int(sa.item()) == int(sb.item()) == 0
             # four stages, sums of fewer than 100 products in another order
             assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
+
+
+@pytest.mark.parametrize('sites,modes,subspace', [(5, 2, 'ge'), (6, 1, 'ge')])
+def test_crowded_batches_of_few_modes(gpu, sites, modes, subspace):
+    """Many right-hand sides of six and seven states with few modes take the
+    element-wise kernel (bit by bit), fewer the column form (to rounding)."""
+    eom = _eom(sites, modes, subspace)
+    general = copy.copy(eom)
+    general.flags = eom.flags & 3
+    dev = eom.H.device
+    rs = np.random.RandomState(7)
+    nsub = torch.tensor([2], dtype=torch.int32, device=dev)
+    h = torch.tensor([0.4], dtype=torch.float64, device=dev)
+    for members in (300, 800):
+        y0 = rs.normal(size=(members, 1, eom.size)) + 1j * rs.normal(size=(members, 1, eom.size))
+        y0 = torch.as_tensor(y0).to(dev)
+        a, sa = _native.zofe_propagate(eom, y0, nsub, h)
+        b, sb = _native.zofe_propagate(general, y0, nsub, h)
+        assert int(sa.item()) == int(sb.item()) == 0
+        assert torch.equal(a, b) if members == 800 else \
+            float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
