@@ -48,6 +48,7 @@
 #include "qsx_common.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 #include <vector>
@@ -596,21 +597,24 @@ __global__ void heom_save_kernel(const double2* __restrict__ y, int n_ado, int M
   if (!cfinite(v)) status[0] = 1;
 }
 
-// Samples per pass: the whole hierarchy of a pass (y, ynew and the two stage
-// vectors) is kept small enough to stay largely resident in the 256 MB
-// memory-attached last-level cache while all its steps run, so the stage
-// vectors and the neighbour gathers are served from there instead of HBM;
-// a multiple of the XCD count so that every XCD holds whole samples.
-// QSX_HEOM_SAMPLES_PER_PASS overrides the choice (0 = all samples at once).
+// Samples per pass: the whole hierarchy of a pass (the state y and three terms
+// or stage vectors, see heom_bytes_per_element) is kept small enough to stay
+// largely resident in the 256 MB memory-attached last-level cache while all its
+// steps run, so the terms and the neighbour gathers are served from there
+// instead of HBM; a multiple of the XCD count so that every XCD holds whole
+// samples.  QSX_HEOM_SAMPLES_PER_PASS overrides the choice (0 = all samples at
+// once).
 inline int heom_samples_per_pass(int B, int64_t bytes_per_sample) {
   const char* env = getenv("QSX_HEOM_SAMPLES_PER_PASS");
   if (env != nullptr) {
     const int v = atoi(env);
     return v <= 0 ? B : std::min(B, v);
   }
-  // measured on the 7-site, 3060-ADO hierarchy (MI355X): passes of 24
-  // samples are the fastest in FP64 (9.6 MB each) and within 2% of the
-  // fastest in MIXED (10.8 MB each); 48 are 20-25% slower in both
+  // measured, 20 steps of 7-site, 3060-ADO hierarchies: 48 samples in FP64 (9.6
+  // MB each, the budget's passes of 24) 7.9 ms in passes of 24, 8.2, 8.7 and 8.4
+  // in 32, 40 and 48; in MIXED (6.0 MB, passes of 40 and 8) 7.4, and 7.6, 7.4 and
+  // 7.1 in 24, 32 and 48; 96 samples in MIXED 14.2 (40, 40, 16), 14.1 in passes
+  // of 48 and 15.4 in one
   const int64_t budget = 260ll << 20;
   int c = (int)std::max<int64_t>(1, budget / std::max<int64_t>(1, bytes_per_sample));
   if (c >= kXcds) c -= c % kXcds;
@@ -624,17 +628,19 @@ inline void set_tile(HeomArgs& a, int elems) {
 
 // Elements per thread (1 .. kElemsPerThread) for launches of B samples: the
 // fewest rounds of work-groups on the chip, each priced at its elements per
-// thread and half an element for the operators and tables it sets up.  Returns
-// the kernel's dynamic LDS bytes.
+// thread and half an element for the operators and tables it sets up (beyond
+// three rounds work-groups of neighbouring rounds overlap, and half of the last
+// round's idle part is not counted).  Returns the kernel's dynamic LDS bytes.
 // Measured (20 steps, us FP64 / MIXED at three, two and one): 7 sites, 3060 ADOs,
 // 4 samples (0.5, 0.8, 1.6 rounds) 1210 / 1290, 1165 / 1120, 1240 / 1150; 8
-// samples (1.1, 1.6, 3.2) 1870 / 1735, 1705 / 1660 (two); 2024 ADOs, two terms, 4
-// samples (0.4, 0.6, 1.3) 1250 / 1440, 985 / 1120, 1010 / 1035, 8 samples (0.8,
-// 1.3, 2.5) 1310 / 1310, 1485 / 1425, 1375 / 1370; 5 sites, 1001 ADOs, 48
-// samples (1.1, 1.6, 3.2) 1840 / 1635, 1565 / 1460 (two).  One element per thread
-// only below 512 work-groups, as before, took three for all of these.
+// samples (1.1, 1.6, 3.2) 1870 / 1735, 1705 / 1660 (two); 40 samples (5.3, 8.0 of
+// which the last is full) MIXED 7455, 7620; 2024 ADOs, two terms, 4 samples (0.4,
+// 0.6, 1.3) 1250 / 1440, 985 / 1120, 1010 / 1035, 8 samples (0.8, 1.3, 2.5) 1310 /
+// 1310, 1485 / 1425, 1375 / 1370; 5 sites, 1001 ADOs, 48 samples (1.1, 1.6, 3.2)
+// 1840 / 1635, 1565 / 1460 (two).  One element per thread only below 512
+// work-groups took three for all of these.
 inline size_t choose_tile(HeomArgs& a, int B, const void* kern, size_t elem_bytes) {
-  int64_t best = INT64_MAX;
+  double best = INFINITY;
   int pick = kElemsPerThread;
   for (int elems = kElemsPerThread; elems >= 1; --elems) {
     set_tile(a, elems);
@@ -643,8 +649,8 @@ inline size_t choose_tile(HeomArgs& a, int B, const void* kern, size_t elem_byte
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kThreads, lds) != hipSuccess)
       (void)hipGetLastError();
     if (per_cu < 1) break;              // the launch's own checks report it
-    const int64_t slots = (int64_t)kCUs * per_cu;
-    const int64_t cost = ((int64_t)B * a.tiles + slots - 1) / slots * (2 * elems + 1);
+    const double r = (double)B * a.tiles / (kCUs * per_cu);
+    const double cost = (r > 3 ? 0.5 * (r + std::ceil(r)) : std::ceil(r)) * (elems + 0.5);
     if (cost < best) {
       best = cost;
       pick = elems;
