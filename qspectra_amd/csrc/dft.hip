@@ -24,17 +24,17 @@
 // one complex multiply-add per sample) and R = 1, 2 or 4 batch rows (the
 // twiddles are the rows'): 4 + 4 / R FP64 operations per sample for two
 // outputs, where one output of one row took 8.  The rows are staged through
-// LDS in tiles (every thread reads the same sample: broadcast), 8 KB per
-// work-group whatever R, and a launch has threads for the pairs that have an
-// output only, in work-groups of whole wavefronts: short grids (up to 127
-// points: one wavefront) and the adjoints of short signals far from t = 0 keep
-// twenty work-groups on a CU.  Four chains of twiddles, each advanced by four
-// samples' step, hide their latency.
-// Measured (host call): 129 rows of 1000 samples onto 1999 points 67 us, with
+// LDS in tiles (every thread reads the same sample: broadcast), 8 or 16 KB per
+// work-group, and a launch has threads for the pairs that have an
+// output only, where they fill the chip in work-groups of whole wavefronts:
+// short grids (up to 127 points: one wavefront) and the adjoints of short signals
+// far from t = 0 keep up to twenty work-groups on a CU.  Four chains of
+// twiddles, each advanced by four samples' step, hide their latency.
+// Measured (host call): 129 rows of 1000 samples onto 1999 points 63 us, with
 // one output of one row per thread 122 us; 20000 rows of 61 samples onto 121
-// points 26 us, the adjoint 41 us, with N / 2 + 1 pairs in work-groups of 256
+// points 26 us, the adjoint 39 us, with N / 2 + 1 pairs in work-groups of 256
 // and 32 KB of samples 64 and 112 us, with one output per thread 76 and 94 us;
-// adjoint of 3000 rows from 4000 points to 100 samples at their end 446, 4402
+// adjoint of 3000 rows from 4000 points to 100 samples at their end 443, 4306
 // and 677 us.
 //
 // Long transforms (both lengths >= kChirpMin) take Bluestein's chirp-z form
@@ -69,8 +69,10 @@ namespace qsx {
 namespace {
 
 constexpr int kDftThreads = 256;
-constexpr int kDftTile = 512;  // samples in LDS, of all R rows together
-constexpr int kAnchor = 16;   // samples between exact twiddles (divides kDftTile / R)
+constexpr int kAnchor = 16;   // samples between exact twiddles (divides a tile)
+// samples per row in LDS: 8 KB for four rows, whose launches fill the chip (also
+// with work-groups of one wavefront), 8 and 16 KB for one and two
+constexpr int dft_tile(int R) { return R == 4 ? 128 : 512; }
 
 __global__ __launch_bounds__(kDftThreads) void dft_twiddle_kernel(int N, double2* __restrict__ T) {
   const int m = blockIdx.x * kDftThreads + threadIdx.x;
@@ -95,9 +97,9 @@ __global__ __launch_bounds__(kDftThreads) void dft_kernel(
     const double2* __restrict__ in, int64_t batch, int n_in, int n_out, int N, int64_t a0,
     int da, int64_t d0, int dd, int q0, int nq, int adj, double scale,
     const double2* __restrict__ T, double2* __restrict__ out) {
-  constexpr int kTile = kDftTile / R;
+  constexpr int kTile = dft_tile(R), U = 2;
   __shared__ double2 xs[R][kTile];
-  const int nt = blockDim.x;
+  const int nt = R == 4 ? blockDim.x : kDftThreads;
   const int64_t q = (int64_t)blockIdx.x * nt + threadIdx.x;
   const bool mine = q < nq, busy = __any(mine);
   const int64_t a = q0 + min(q, (int64_t)(nq - 1));
@@ -117,10 +119,27 @@ __global__ __launch_bounds__(kDftThreads) void dft_kernel(
     for (int v0 = 0; v0 < n_in; v0 += kTile) {
       const int len = min(kTile, n_in - v0);
       __syncthreads();
+      if constexpr (R == 2) {         // R U loads in flight (129 rows as above: 63 us for 66)
+        for (int k0 = threadIdx.x; k0 < len; k0 += U * nt) {
+          double2 x[R][U];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const double2* row = in + min(b0 + r, batch - 1) * n_in + v0;
-        for (int k = threadIdx.x; k < len; k += nt) xs[r][k] = row[k];
+          for (int r = 0; r < R; ++r) {
+            const double2* row = in + min(b0 + r, batch - 1) * n_in + v0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[r][u] = row[min(k0 + u * nt, len - 1)];
+          }
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (k0 + u * nt < len) xs[r][k0 + u * nt] = x[r][u];
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const double2* row = in + min(b0 + r, batch - 1) * n_in + v0;
+          for (int k = threadIdx.x; k < len; k += nt) xs[r][k] = row[k];
+        }
       }
       __syncthreads();
       // exact twiddle from the table every kAnchor samples, in between multiplied
@@ -770,12 +789,14 @@ extern "C" int32_t qsx_fourier_transform(const void* x, int64_t batch, int32_t n
   const int64_t amin = std::min(a0, a1), amax = std::max(a0, a1);
   const int q0 = (int)(amin > 0 ? amin : (amax < 0 ? -amax : 0));
   const int nq = (int)std::max(-amin, amax) - q0 + 1;
-  // equal work-groups of whole wavefronts; more rows per thread while that
-  // leaves two wavefronts (four rows) or one (two rows) for every SIMD
+  // more rows per thread while that leaves two wavefronts (four rows) or one (two
+  // rows) for every SIMD; work-groups of as few wavefronts as the pairs need
+  // where they fill the chip, else all 256 threads stage the samples
   const int64_t gx = (nq + kDftThreads - 1) / kDftThreads;
-  const int waves = (int)(((nq + gx - 1) / gx + 63) / 64);
+  int waves = (int)(((nq + gx - 1) / gx + 63) / 64);
   const int R = gx * waves * ((batch + 3) / 4) >= 2048 ? 4
               : (gx * waves * ((batch + 1) / 2) >= 1024 ? 2 : 1);
+  if (R < 4) waves = kDftThreads / 64;
   const auto kern = R == 4 ? dft_kernel<4> : (R == 2 ? dft_kernel<2> : dft_kernel<1>);
   const unsigned gy = (unsigned)std::min<int64_t>((batch + R - 1) / R, 65535);
   hipLaunchKernelGGL(kern, dim3((unsigned)gx, gy), dim3(64 * waves), 0, s,
