@@ -394,10 +394,11 @@ __global__ __launch_bounds__(NT) void zofe_kernel(ZofeArgs a, const double2* __r
 //       element of rho, one term of its sums per lane, those over sites again
 //       only over the sites that couple;
 //   (3) the RK4 update written back into LDS.
-// Measured (7 sites, 16 modes, one right-hand side): 8.2 us per stage, with
-// the element-wise kernel 16.2 us (its LDS reads, phases and workspace round
-// trips).  Of the 8.2 us, (2) takes 5.8 us, two wavefronts per SIMD in FP64
-// multiply-adds at 73% of their issue rate; (1) and (3) are latency.
+// Measured (7 sites, 16 modes, one right-hand side): 7.7 us per stage (kernel
+// trace: 100 steps 3.09 ms), with the element-wise kernel 16.2 us (its LDS reads,
+// phases and workspace round trips).  The 784 FP64 multiply-adds of a thread in
+// (2), two wavefronts per SIMD, are 2.6 us of issue at 2.4 GHz; the rest is
+// latency: LDS reads and broadcasts between them, (1), (3) and the barriers.
 // LDS: a thread's columns are NC apart and the blocks start 16 banks apart
 // (4 entries modulo 16), so that the 16 lanes of an access, NC neighbouring
 // columns of 16 / NC blocks, meet different banks.
@@ -809,7 +810,7 @@ static int32_t zofe_launch(int apply,
   // 1300), 1.05 to 3.4 times over 1..8 states and 1..16 modes, one right-hand side
   // or 300.  One column per thread while that takes at most one wavefront per
   // SIMD, two beyond (each row of X then read once for both; one column in 128
-  // registers measured 13.2 us per stage against 8.2 us).  At 6 and 7 states it
+  // registers measured 13.2 us per stage, two 7.7).  At 6 and 7 states it
   // holds one work-group per CU (122 and 147 us per 256 right-hand sides and 8
   // steps) where the element-wise kernel with few modes holds up to four: from
   // two to four rounds on that one is taken (8 steps, 1024 right-hand sides, column /
