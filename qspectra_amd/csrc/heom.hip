@@ -350,9 +350,11 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // Measured (7 sites, 3060 ADOs, per stage of 24 samples): 49 us FP64, 47 us
 // MIXED; 74 and 66 us when every edge was gathered, all products were complex
 // and stages wrote separate stage vectors (55 and 62 us with the existing
-// edges alone).  In FP64 a stage now moves 210 MB (FETCH_SIZE, WRITE_SIZE) at
-// 4.3 TB/s, where a device copy reaches 5.1.  Nested brackets y + h/m A (..)
-// in place of the series terms and non-temporal loads and stores were slower.
+// edges alone).  In FP64 a stage moves 204 MB (FETCH_SIZE, WRITE_SIZE) at 4.2
+// TB/s, where a device copy reaches 5.1; in MIXED one of 40 samples 227 MB in 79
+// us, 2.9 TB/s, with the vector ALUs issuing 48% of the time: latency of the
+// gathers.  Nested brackets y + h/m A (..) in place of the series terms and
+// non-temporal loads and stores were slower.
 // TIN: the type of the stage's input (MIXED: double for the series' first
 // stage, whose input is y).
 //
