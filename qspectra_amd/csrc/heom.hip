@@ -351,8 +351,8 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // MIXED; 74 and 66 us when every edge was gathered, all products were complex
 // and stages wrote separate stage vectors (55 and 62 us with the existing
 // edges alone).  In FP64 a stage moves 204 MB (FETCH_SIZE, WRITE_SIZE) at 4.2
-// TB/s, where a device copy reaches 5.1; in MIXED one of 40 samples 227 MB in 79
-// us, 2.9 TB/s, with the vector ALUs issuing 48% of the time: latency of the
+// TB/s, where a device copy reaches 5.1; in MIXED one of 40 samples 227 MB in 76
+// us, 3.0 TB/s, with the vector ALUs issuing 48% of the time: latency of the
 // gathers.  Nested brackets y + h/m A (..) in place of the series terms and
 // non-temporal loads and stores were slower.
 // TIN: the type of the stage's input (MIXED: double for the series' first

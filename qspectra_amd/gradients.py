@@ -314,7 +314,7 @@ class RedfieldAbsorption(object):
         H1 = self.hamiltonians(E, J)
         L = self.liouvillian(H1, lam)
         P = rk4_propagator(L, self.dt)
-        if self._pieces is not None:
+        if self._pieces is not None and not self.v.requires_grad:
             x, status = _PropagatePieces.apply(P, self.y0, self._pieces, self.v)
             if int(status.item()) == 0:
                 return x[:, 0].mean(dim=0)

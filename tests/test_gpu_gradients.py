@@ -10,6 +10,7 @@ import torch
 import qspectra_amd as qa
 from qspectra_amd import _native
 from qspectra_amd import gradients as G
+from qspectra_amd import workloads as W
 from oracle import system as S
 from oracle import liouville as Lv
 from oracle import propagate as P
@@ -333,3 +334,21 @@ def test_records_across_widths(gpu, n):
         ref = (Ht.grad[0] + Ht.grad[0].T).numpy() / 2
         assert np.abs(gH[b].cpu().numpy() - ref).max() < 1e-9 * np.abs(ref).max()
         assert abs(float(glam[b]) - float(lam.grad)) < 1e-9 * abs(float(lam.grad))
+
+
+def test_signal_vector_keeps_its_gradient(gpu):
+    """A signal vector that is differentiated is contracted with the states:
+    its gradient equals that of the explicit contraction."""
+    H, d, _ = W.aggregate7_hamiltonian()
+    spec = G.RedfieldAbsorption(d, 106.0, BATH[0], 12450.0, 200.0, 1.0)
+    E = torch.tensor(np.diag(H).copy(), device='cuda')
+    J = torch.tensor(H[np.triu_indices(7, 1)], device='cuda')
+    plain = spec.signal(E, J, 35.0)
+    spec.v = spec.v.clone().requires_grad_(True)
+    x = spec.signal(E, J, 35.0)
+    assert rel_err(x.detach().cpu().numpy(), plain.cpu().numpy()) < 1e-12
+    (x.abs() ** 2).sum().backward()
+    P = G.rk4_propagator(spec.liouvillian(spec.hamiltonians(E, J), 35.0), spec.dt)
+    y = G.propagate(P, spec.y0, spec.nsub)[0, 0]
+    want = 2 * (y.conj() * x.detach()[:, None]).sum(dim=0)
+    assert rel_err(spec.v.grad.cpu().numpy(), want.cpu().numpy()) < 1e-12

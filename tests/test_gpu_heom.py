@@ -304,3 +304,29 @@ def test_ensemble_of_a_model_that_has_been_used(gpu):
             qa.simulate_dynamics(m, rho0, times=t, dt=0.5)
         out.append(qa.simulate_dynamics(m, rho0, times=t, ensemble_size=3, dt=0.5)[1])
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+def test_heom_propagation_under_capture(gpu, precision):
+    """A captured propagation replays the eager one bit by bit, with eager
+    work between the replays (the launch shape comes from a host query)."""
+    m = _model('redfield_7site', rw=float(golden('heom')['agg7_rw_freq']))
+    eom = m.with_hamiltonians([m.hamiltonian.sample(n) for n in range(3)]).equation_of_motion('ee')
+    rs = np.random.RandomState(0)
+    y0 = torch.as_tensor(rs.normal(size=(3, eom.size)) + 1j * rs.normal(size=(3, eom.size))).cuda()
+    mode = _native.QSX_FP64 if precision == 'fp64' else _native.QSX_MIXED
+
+    def go():
+        return _native.heom_propagate(eom, y0, [2, 3], [0.5, 0.25], mode)[0]
+    want = go()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = go()
+    for scale in (1.0, -2.0, 0.5):
+        y0.mul_(scale)
+        want = go()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
