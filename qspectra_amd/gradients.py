@@ -171,8 +171,9 @@ def propagate(A, y0, nsub, ckpt=64):
     """Differentiable propagation with the one-step propagator A [B|1, M, M]:
     states [B, R, len(nsub), M] (nsub: host step counts per save interval).
     The reverse pass recomputes the forward states from checkpoints every
-    ckpt steps (blocks up to M = 160; at most 16 states: from the starts of
-    the pieces the steps are cut into, see _native.PieceSchedule)."""
+    ckpt steps (blocks up to M = 160), or where _pieces takes the call (at most
+    16 states, long recursions) from the starts of the pieces the steps are cut
+    into."""
     grad = torch.is_grad_enabled() and (A.requires_grad or y0.requires_grad)
     sched = _pieces(y0.shape[-1], y0.shape[0] * y0.shape[1], nsub, y0.device, grad=grad)
     if sched is not None:
