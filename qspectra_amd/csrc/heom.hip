@@ -644,18 +644,25 @@ inline void set_tile(HeomArgs& a, int elems) {
 inline size_t choose_tile(HeomArgs& a, int B, const void* kern, size_t elem_bytes) {
   double best = INFINITY;
   int pick = kElemsPerThread;
-  for (int elems = kElemsPerThread; elems >= 1; --elems) {
-    set_tile(a, elems);
-    const size_t lds = heom_lds_bytes(heom_opsz(a), a.ado_per_tile, a.M, a.nbins, elem_bytes, a.N);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kThreads, lds) != hipSuccess)
-      (void)hipGetLastError();
-    if (per_cu < 1) break;              // the launch's own checks report it
-    const double r = (double)B * a.tiles / (kCUs * per_cu);
-    const double cost = (r > 3 ? 0.5 * (r + std::ceil(r)) : std::ceil(r)) * (elems + 0.5);
-    if (cost < best) {
-      best = cost;
-      pick = elems;
+  set_tile(a, 1);
+  if ((int64_t)B * a.tiles <= kCUs) {
+    pick = 1;         // one round whatever the occupancy, which takes longer to ask
+  } else {            // for than a small hierarchy's step
+    for (int elems = 1; elems <= kElemsPerThread; ++elems) {
+      set_tile(a, elems);
+      const size_t lds = heom_lds_bytes(heom_opsz(a), a.ado_per_tile, a.M, a.nbins, elem_bytes,
+                                        a.N);
+      int per_cu = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kThreads, lds) != hipSuccess)
+        (void)hipGetLastError();
+      if (per_cu < 1) break;            // the launch's own checks report it
+      const double r = (double)B * a.tiles / (kCUs * per_cu);
+      const double cost = (r > 3 ? 0.5 * (r + std::ceil(r)) : std::ceil(r)) * (elems + 0.5);
+      if (cost <= best) {
+        best = cost;
+        pick = elems;
+      }
+      if (r <= 1) break;                // more elements only lengthen the round
     }
   }
   set_tile(a, pick);
