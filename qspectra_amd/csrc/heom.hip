@@ -343,7 +343,16 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // c_k n_j(r) - conj(c_k) n_j(c)) tabulated once per work-group.
 // Three quarters of the (ADO, bin, kind) edges of a truncated hierarchy do not
 // exist (no upward ones at the last level, downward ones only from occupied
-// bins): their gathers, coefficients and products are skipped lane by lane.
+// bins): from 4 states their gathers, coefficients and products are skipped
+// lane by lane.  At 2 and 3 states they gather the element's own value with their
+// zero coefficient instead: most of those hierarchies have fewer work-groups than
+// the device has CUs, a stage lasts as long as one element's chain, and a branch
+// per edge puts its coefficient's LDS read behind the branch before it.  20 steps
+// of 1 sample, branches -> none: 2 sites, 28 ADOs, two terms 428 -> 383 us FP64,
+// 471 -> 386 MIXED; 3 sites, 715 ADOs, two terms 510 -> 466 and 601 -> 455.
+// Where the device is full it gains in MIXED and loses in FP64: 400 samples of 3
+// sites, 1716 ADOs 6.5 -> 6.8 ms FP64, 5.8 -> 5.5 MIXED; 210 ADOs of a complex
+// Hamiltonian 1.42 -> 1.23 and 1.52 -> 1.03.
 // Purely imaginary operators (-i unit H of a real H, -i unit times a real
 // edge coefficient) take half the multiply-adds; the form is decided per
 // work-group from the entries it has loaded.
@@ -363,14 +372,16 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // column in registers: at 8 states 4 wavefronts per SIMD for one Matsubara term
 // and 3 for two leave room for that (132 and 140 registers), and it is the
 // fastest; below, the element index is kept opaque so that the entries stay in
-// LDS and 6 (5) wavefronts fit in 80 (96) registers with at most 4 spilled.
+// LDS and, from 4 states, 6 (5) wavefronts fit in 80 (96) registers with at most 4
+// spilled.  2 and 3 states need at most 87 registers with all gathers in flight;
+// their bound of 3 only keeps the compiler from serialising them.
 // Measured against one bound of 6 (4 for two terms) at every size: 8 sites, 969
 // ADOs, 48 samples, 20 steps 7.6 -> 3.6 ms FP64 and 6.0 -> 3.6 MIXED for a real
 // Hamiltonian, 3.5 for a complex one (24 samples took 7.7), 75 to 100 registers
 // spilled before; 7 sites, 2024 ADOs, two terms 7.0 -> 6.0 and 5.8 -> 5.5; 7
 // sites, one term unchanged.
 constexpr int comm_waves(int nX, int kb) {
-  return nX == 8 ? (kb == 2 ? 4 : 3) : (kb == 2 ? 6 : 5);
+  return nX <= 3 ? 3 : nX == 8 ? (kb == 2 ? 4 : 3) : (kb == 2 ? 6 : 5);
 }
 
 template <typename T, typename TIN, int NX, int NY, int NR, int KB>
@@ -444,7 +455,8 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
     constexpr bool GENERAL = decltype(form)::value;
     // gathers in flight: of all slots where the registers allow it (the small
     // hierarchies of 2 and 3 states wait for their latency), else of one
-    constexpr int SLOTS = NX <= 3 ? NR : 1;
+    constexpr bool FLAT = NX <= 3;               // no branches on absent edges
+    constexpr int SLOTS = FLAT ? NR : 1;
     for (int e = tid; e < nloc * M; e += kThreads) {
       int eo = e;
       if (NX < 8) asm volatile("" : "+v"(eo));     // see the registers above
@@ -470,7 +482,8 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
 #pragma unroll
         for (int o = 0; o < 2 * KB; ++o) {
           v[u][o] = T2{0, 0};
-          if (src[u][o] >= 0) v[u][o] = zb[src[u][o] * M + p];
+          if (FLAT) v[u][o] = zb[(src[u][o] >= 0 ? src[u][o] : ado) * M + p];
+          else if (src[u][o] >= 0) v[u][o] = zb[src[u][o] * M + p];
         }
       };
       if (SLOTS > 1)
@@ -499,7 +512,7 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
         }
 #pragma unroll
         for (int o = 0; o < 2 * KB; ++o) {
-          if (src[u][o] >= 0) {
+          if (FLAT || src[u][o] >= 0) {
             const double2 cf = tc[pbin[p][t] + o], x = to_d2(v[u][o]);
             if (o % 2 == 0) {
               const double w = pwp[p][t];
