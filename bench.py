@@ -435,10 +435,10 @@ HEOM_BYTES_PER_ELEMENT_STEP = {'fp64': 176, 'mixed': 112}
 # launch of several kernels counts all of them.
 PMC_TRAFFIC = {
     # one RK4 stage over 256 members, summed over its sample passes (10 of 24
-    # members and one of 16 in FP64, 6 of 40 and one of 16 in MIXED; FP64 56.8 B
-    # per element-stage, MIXED 37.2 B)
-    'heom stage fp64': 2.179e9,
-    'heom stage mixed': 1.427e9,
+    # members and one of 16 in FP64, 6 of 40 and one of 16 in MIXED; FP64 59.1 B
+    # per element-stage, MIXED 39.2 B)
+    'heom stage fp64': 2.268e9,
+    'heom stage mixed': 1.506e9,
     # the headline plan's t2 operator program (one work-group, M = 49)
     'propagate powers M=49 B=1 R=7 e=0,100,200,500': 8.64e4,
     'chunks prop mixed M=147 nc=8 B=1 steps=15 nsave=16': 4.30e6,

@@ -348,7 +348,8 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // zero coefficient instead: most of those hierarchies have fewer work-groups than
 // the device has CUs, a stage lasts as long as one element's chain, and a branch
 // per edge puts its coefficient's LDS read behind the branch before it.  20 steps
-// of 1 sample, branches -> none: 2 sites, 28 ADOs, two terms 428 -> 383 us FP64,
+// of 1 sample, branches -> none (with each table loaded behind the one before, see
+// below): 2 sites, 28 ADOs, two terms 428 -> 383 us FP64,
 // 471 -> 386 MIXED; 3 sites, 715 ADOs, two terms 510 -> 466 and 601 -> 455.
 // Where the device is full it gains in MIXED and loses in FP64: 400 samples of 3
 // sites, 1716 ADOs 6.5 -> 6.8 ms FP64, 5.8 -> 5.5 MIXED; 210 ADOs of a complex
@@ -356,12 +357,12 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // Purely imaginary operators (-i unit H of a real H, -i unit times a real
 // edge coefficient) take half the multiply-adds; the form is decided per
 // work-group from the entries it has loaded.
-// Measured (7 sites, 3060 ADOs, per stage of 24 samples): 49 us FP64, 47 us
+// Measured (7 sites, 3060 ADOs, per stage of 24 samples): 44 us FP64, 44 us
 // MIXED; 74 and 66 us when every edge was gathered, all products were complex
 // and stages wrote separate stage vectors (55 and 62 us with the existing
-// edges alone).  In FP64 a stage moves 204 MB (FETCH_SIZE, WRITE_SIZE) at 4.2
-// TB/s, where a device copy reaches 5.1; in MIXED one of 40 samples 227 MB in 76
-// us, 3.0 TB/s, with the vector ALUs issuing 48% of the time: latency of the
+// edges alone).  In FP64 a stage moves 212 MB (FETCH_SIZE, WRITE_SIZE) at 4.8
+// TB/s, where a device copy reaches 5.1; in MIXED one of 40 samples 235 MB in 70
+// us, 3.4 TB/s, with the vector ALUs issuing 53% of the time: latency of the
 // gathers.  Nested brackets y + h/m A (..) in place of the series terms and
 // non-temporal loads and stores were slower.
 // TIN: the type of the stage's input (MIXED: double for the series' first
@@ -370,15 +371,15 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // Registers.  Where M divides the work-group (4 and 8 states) a thread's elements
 // share their row and column, and the compiler holds the operator's row and
 // column in registers: at 8 states 4 wavefronts per SIMD for one Matsubara term
-// and 3 for two leave room for that (132 and 140 registers), and it is the
-// fastest; below, the element index is kept opaque so that the entries stay in
+// and 3 for two leave room for that (128 registers and 4 spilled, at most
+// 140), and it is the fastest; below, the element index is kept opaque so that the entries stay in
 // LDS and, from 4 states, 6 (5) wavefronts fit in 80 (96) registers with at most 4
 // spilled.  2 and 3 states need at most 87 registers with all gathers in flight;
 // their bound of 3 only keeps the compiler from serialising them.
 // Measured against one bound of 6 (4 for two terms) at every size: 8 sites, 969
 // ADOs, 48 samples, 20 steps 7.6 -> 3.6 ms FP64 and 6.0 -> 3.6 MIXED for a real
-// Hamiltonian, 3.5 for a complex one (24 samples took 7.7), 75 to 100 registers
-// spilled before; 7 sites, 2024 ADOs, two terms 7.0 -> 6.0 and 5.8 -> 5.5; 7
+// Hamiltonian, 3.5 for a complex one (24 samples took 7.7; all 3.3 to 3.4 now), 75
+// to 100 registers spilled before; 7 sites, 2024 ADOs, two terms 7.0 -> 6.0 and 5.8 -> 5.5; 7
 // sites, one term unchanged.
 constexpr int comm_waves(int nX, int kb) {
   return nX <= 3 ? 3 : nX == 8 ? (kb == 2 ? 4 : 3) : (kb == 2 ? 6 : 5);
@@ -420,30 +421,56 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
   const int64_t base = ((int64_t)b * a.n_ado + ado0) * M;
   const double2* Hb = a.Hop + (int64_t)b * OPSZ;
   bool general = false;                      // operators not purely imaginary
-  for (int e = tid; e < OPSZ; e += kThreads) {
-    Hs[e] = Hb[e];
-    general |= Hs[e].x != 0.0;
+  // The first trips of the four tables are loaded together, and the tables' loads
+  // depend on no earlier one (the coefficient of an absent edge is loaded too, as
+  // are the pads' occupations): with each table's loads behind the table before,
+  // seven latencies in a row, 20 steps took 1.05 to 1.14 times as long at 2 states
+  // (28 ADOs, 1 sample 375 -> 342 us FP64, 380 -> 356 MIXED), 1.02 to 1.15 at 7 (48
+  // samples, 3060 ADOs 7.86 -> 7.19 ms and 7.45 -> 6.95), 1.02 to 1.10 at 8.
+  // Later trips load for themselves: with the next trip's values held in registers
+  // the compiler wrote a source index over the low half of a coefficient.
+  const T2* zt0 = zin + base;
+  const int* sb = a.bsrc + (int64_t)ado0 * nb2;
+  const double2* cb = a.bcoef + (int64_t)ado0 * nb2;
+  double2 hv = make_double2(0.0, 0.0), zv = hv, cv = hv;
+  int sv = -1, jv = -1;
+  double2 ov = hv, ck[KB];
+  if (tid < OPSZ) hv = Hb[tid];
+  if (tid < nloc * M) zv = ld<TIN>(zt0 + tid);
+  if (tid < nloc * nb2) {
+    sv = sb[tid];
+    cv = cb[tid];
   }
-  for (int e = tid; e < nloc * M; e += kThreads) zt[e] = ld<TIN>(zin + base + e);
-  for (int e = tid; e < nloc * nb2; e += kThreads) {
-    const int64_t g = (int64_t)ado0 * nb2 + e;
-    const int src = a.bsrc[g];
+  if (tid < M * NR) {
+    jv = a.rsite[tid];
+    ov = make_double2(a.rocc[2 * tid], a.rocc[2 * tid + 1]);
+  }
+#pragma unroll
+  for (int kk = 0; kk < KB; ++kk) ck[kk] = a.ck[kk];
+  static_assert(OPSZ <= kThreads && M * NR <= kThreads, "one trip");
+  if (tid < OPSZ) {
+    Hs[tid] = hv;
+    general |= hv.x != 0.0;
+  }
+  if (tid < nloc * M) zt[tid] = zv;
+  auto edge = [&](int e, int src, double2 cf) {
     const bool ok = src >= 0 && src < a.n_ado;
     tsrc[e] = ok ? src : -1;
-    tcf[e] = ok ? a.bcoef[g] : make_double2(0.0, 0.0);
+    tcf[e] = ok ? cf : make_double2(0.0, 0.0);
     general |= tcf[e].x != 0.0;
-  }
-  for (int e = tid; e < M * NR; e += kThreads) {
-    const int p = e / NR, t = e % NR;
-    const int j = a.rsite[p * NR + t];
-    const bool okj = j >= 0 && (j + 1) * KB <= a.nbins;
-    const double orow = okj ? a.rocc[(p * NR + t) * 2] : 0.0;
-    const double ocol = okj ? a.rocc[(p * NR + t) * 2 + 1] : 0.0;
-    pbin[p][t] = okj ? 2 * j * KB : 0;
+  };
+  if (tid < nloc * nb2) edge(tid, sv, cv);
+  for (int e = tid + kThreads; e < nloc * M; e += kThreads) zt[e] = ld<TIN>(zt0 + e);
+  for (int e = tid + kThreads; e < nloc * nb2; e += kThreads) edge(e, sb[e], cb[e]);
+  if (tid < M * NR) {
+    const int p = tid / NR, t = tid % NR;
+    const bool okj = jv >= 0 && (jv + 1) * KB <= a.nbins;
+    const double orow = okj ? ov.x : 0.0, ocol = okj ? ov.y : 0.0;
+    pbin[p][t] = okj ? 2 * jv * KB : 0;
     pwp[p][t] = orow - ocol;
 #pragma unroll
     for (int kk = 0; kk < KB; ++kk) {
-      const double2 c = a.ck[kk];
+      const double2 c = ck[kk];
       pwm[p][t][kk] = make_double2(c.x * orow - c.x * ocol, c.y * orow + c.y * ocol);
     }
   }
@@ -457,7 +484,13 @@ __global__ __launch_bounds__(kThreads, comm_waves(NX, KB)) void heom_comm_kernel
     // hierarchies of 2 and 3 states wait for their latency), else of one
     constexpr bool FLAT = NX <= 3;               // no branches on absent edges
     constexpr int SLOTS = FLAT ? NR : 1;
-    for (int e = tid; e < nloc * M; e += kThreads) {
+    // the thread's offset is computed here again: kept from the tables' loads, two
+    // registers per thread were spilled at 7 states (MIXED, 48 samples 6.95 -> 7.22
+    // ms); at 8 states it would move the operator's row and column to LDS (969 ADOs,
+    // 48 samples 3.3 -> 4.0 ms)
+    int e0 = tid;
+    if (NX < 8) asm volatile("" : "+v"(e0));       // see the registers above
+    for (int e = e0; e < nloc * M; e += kThreads) {
       int eo = e;
       if (NX < 8) asm volatile("" : "+v"(eo));     // see the registers above
       const int la = eo / M, p = eo - la * M, ado = ado0 + la;
