@@ -371,11 +371,12 @@ __global__ __launch_bounds__(kThreads) void heom_stage_kernel(
 // Registers.  Where M divides the work-group (4 and 8 states) a thread's elements
 // share their row and column, and the compiler holds the operator's row and
 // column in registers: at 8 states 4 wavefronts per SIMD for one Matsubara term
-// and 3 for two leave room for that (128 registers and 4 spilled, at most
-// 140), and it is the fastest; below, the element index is kept opaque so that the entries stay in
-// LDS and, from 4 states, 6 (5) wavefronts fit in 80 (96) registers with at most 4
-// spilled.  2 and 3 states need at most 87 registers with all gathers in flight;
-// their bound of 3 only keeps the compiler from serialising them.
+// and 3 for two leave room for that (128 registers and 4 spilled, at most 140),
+// and it is the fastest; below, the element index is kept opaque so that the
+// entries stay in LDS and, from 4 states, 6 (5) wavefronts fit in 80 (96) registers
+// with at most 4 spilled.  2 and 3 states need at most 87 registers with all
+// gathers in flight; their bound of 3 only keeps the compiler from serialising
+// them.
 // Measured against one bound of 6 (4 for two terms) at every size: 8 sites, 969
 // ADOs, 48 samples, 20 steps 7.6 -> 3.6 ms FP64 and 6.0 -> 3.6 MIXED for a real
 // Hamiltonian, 3.5 for a complex one (24 samples took 7.7; all 3.3 to 3.4 now), 75
